@@ -557,6 +557,23 @@ int spc_sparse_conv_classes(spc_stream_t stream, int dtype, const void* x, const
                             int64_t n_out, int64_t n_in, int64_t cin, int64_t cout,
                             int64_t class_rows, int64_t n_classes, const spc_conv_epilogue* epi);
 
+/* The 27-tap conv of spc_sparse_conv_fused over a table whose output rows
+ * share few source rows (an upsampled level's fine rows over its coarse
+ * rows): P = W_o x[r] for every source row and tap, F32, then every output
+ * row adds its present taps' products in ascending tap order onto the bias,
+ * rounds once and runs the epilogue -- spc_sparse_conv_fused's values up to
+ * the order of F32 additions.  dtype SPC_BF16 or SPC_F16; w packed
+ * (spc_conv_pack_weights, 27 taps, same dtype); idx token-major [n_out, 27]
+ * (entries outside [0, n_in) are missing taps); cin a multiple of 64, cout
+ * of 32 (NORM_MOD_SILU: 32, 64 or 128).  x, w, y and workspace 16-byte
+ * aligned; workspace holds the products
+ * (spc_conv_products_workspace_bytes: n_in * 27 * cout floats). */
+size_t spc_conv_products_workspace_bytes(int64_t n_in, int64_t cout);
+int spc_sparse_conv_products(spc_stream_t stream, int dtype, const void* x, const void* w,
+                             const void* bias, void* y, const int32_t* idx, int64_t n_out,
+                             int64_t n_in, int64_t cin, int64_t cout, const spc_conv_epilogue* epi,
+                             void* workspace, size_t workspace_bytes);
+
 #ifdef __cplusplus
 }
 #endif

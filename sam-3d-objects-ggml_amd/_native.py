@@ -113,6 +113,10 @@ def lib() -> ctypes.CDLL:
     L.spc_sparse_conv_fused.argtypes = [_P, _INT, _P, _INT, _INT, _P, _P, _P, _P, _P, _INT, _P,
                                         _P, _I64, _I64, _I64, _I64, _I64,
                                         ctypes.POINTER(ConvEpilogue)]
+    L.spc_conv_products_workspace_bytes.restype = _SZ
+    L.spc_conv_products_workspace_bytes.argtypes = [_I64, _I64]
+    L.spc_sparse_conv_products.argtypes = [_P, _INT, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64,
+                                           ctypes.POINTER(ConvEpilogue), _P, _SZ]
     _lib = L
     return L
 
@@ -505,6 +509,43 @@ def conv_plan(idx: torch.Tensor | None, *, ntaps: int, n_out: int, n_in: int | N
     return plan
 
 
+def _epilogue(x, n_out, cout, residual, norm_mod, residual_rows):
+    """(spc_conv_epilogue, tensors it points into) of a conv over n_out rows."""
+    epi = ConvEpilogue(EPI_NONE, 0.0, None, None, None, None, 0, None, 0)
+    keep = []
+    if residual is not None and norm_mod is not None:
+        raise ValueError("one epilogue at a time")
+    if residual is not None:
+        residual = residual.contiguous()
+        if residual_rows is not None:
+            residual_rows = residual_rows.to(torch.int32).contiguous()
+            if residual_rows.shape != (n_out,) or residual.dim() != 2 or residual.shape[1] != cout \
+                    or residual.shape[0] < 1 or residual.dtype != x.dtype:
+                raise ValueError("residual_rows must be int32 [n_out] and residual [R >= 1, cout] "
+                                 "in the feature dtype")
+            epi.residual_rows, epi.n_residual = _ptr(residual_rows), residual.shape[0]
+            keep.append(residual_rows)
+        elif residual.shape != (n_out, cout) or residual.dtype != x.dtype:
+            raise ValueError("residual must be [n_out, cout] in the feature dtype")
+        epi.mode, epi.residual = EPI_RESIDUAL, _ptr(residual)
+        keep.append(residual)
+    if norm_mod is not None:
+        scale, shift, coords, eps = norm_mod
+        _need_gpu(scale, shift, coords)
+        scale = scale.to(torch.float32).contiguous()
+        shift = shift.to(torch.float32).contiguous()
+        coords = coords.contiguous()
+        if scale.shape != shift.shape or scale.dim() != 2 or scale.shape[1] != cout:
+            raise ValueError("scale / shift must be [n_batch, cout]")
+        if coords.dtype != torch.int32 or coords.shape != (n_out, 4):
+            raise ValueError("coords must be int32 [n_out, 4]")
+        epi.mode, epi.eps = EPI_NORM_MOD_SILU, float(eps)
+        epi.scale, epi.shift, epi.coords = _ptr(scale), _ptr(shift), _ptr(coords)
+        epi.n_batch = scale.shape[0]
+        keep += [scale, shift, coords]
+    return epi, keep
+
+
 def sparse_conv(x: torch.Tensor, weight, bias: torch.Tensor | None,
                 idx: torch.Tensor | None, *, ntaps: int, n_out: int,
                 idx_layout: int = IDX_TOKEN_MAJOR, row_perm: torch.Tensor | None = None,
@@ -553,38 +594,7 @@ def sparse_conv(x: torch.Tensor, weight, bias: torch.Tensor | None,
         bias = bias.contiguous()
     if out is None:
         out = torch.empty((n_out, cout), dtype=x.dtype, device=x.device)
-    epi = ConvEpilogue(EPI_NONE, 0.0, None, None, None, None, 0, None, 0)
-    keep = []
-    if residual is not None and norm_mod is not None:
-        raise ValueError("one epilogue at a time")
-    if residual is not None:
-        residual = residual.contiguous()
-        if residual_rows is not None:
-            residual_rows = residual_rows.to(torch.int32).contiguous()
-            if residual_rows.shape != (n_out,) or residual.dim() != 2 or residual.shape[1] != cout \
-                    or residual.shape[0] < 1 or residual.dtype != x.dtype:
-                raise ValueError("residual_rows must be int32 [n_out] and residual [R >= 1, cout] "
-                                 "in the feature dtype")
-            epi.residual_rows, epi.n_residual = _ptr(residual_rows), residual.shape[0]
-            keep.append(residual_rows)
-        elif residual.shape != (n_out, cout) or residual.dtype != x.dtype:
-            raise ValueError("residual must be [n_out, cout] in the feature dtype")
-        epi.mode, epi.residual = EPI_RESIDUAL, _ptr(residual)
-        keep.append(residual)
-    if norm_mod is not None:
-        scale, shift, coords, eps = norm_mod
-        _need_gpu(scale, shift, coords)
-        scale = scale.to(torch.float32).contiguous()
-        shift = shift.to(torch.float32).contiguous()
-        coords = coords.contiguous()
-        if scale.shape != shift.shape or scale.dim() != 2 or scale.shape[1] != cout:
-            raise ValueError("scale / shift must be [n_batch, cout]")
-        if coords.dtype != torch.int32 or coords.shape != (n_out, 4):
-            raise ValueError("coords must be int32 [n_out, 4]")
-        epi.mode, epi.eps = EPI_NORM_MOD_SILU, float(eps)
-        epi.scale, epi.shift, epi.coords = _ptr(scale), _ptr(shift), _ptr(coords)
-        epi.n_batch = scale.shape[0]
-        keep += [scale, shift, coords]
+    epi, keep = _epilogue(x, n_out, cout, residual, norm_mod, residual_rows)  # keep: alive until queued
     if class_rows:
         if not isinstance(weight, PackedWeights):
             raise ValueError("weight classes need PackedWeights")
@@ -599,6 +609,34 @@ def sparse_conv(x: torch.Tensor, weight, bias: torch.Tensor | None,
                                      _ptr(plan), ntaps, n_out, x.shape[0], cin, cout,
                                      ctypes.byref(epi))
     _check("spc_sparse_conv", st)
+    return out
+
+
+def sparse_conv_products(x: torch.Tensor, weight: PackedWeights, bias: torch.Tensor | None,
+                         idx: torch.Tensor, *, n_out: int, norm_mod: tuple | None = None,
+                         residual: torch.Tensor | None = None,
+                         residual_rows: torch.Tensor | None = None) -> torch.Tensor:
+    """The 27-tap conv over a token-major table through per-source-row
+    products (spc_sparse_conv_products); epilogues as in sparse_conv."""
+    _need_gpu(x, bias, idx, weight.data, residual, residual_rows)
+    x = x.contiguous()
+    dt, (n_in, cin), cout = dtype_code(x.dtype), x.shape, weight.cout
+    if weight.ntaps != 27 or weight.cin != cin or weight.w_dtype != dt:
+        raise ValueError("packed weights do not match the features")
+    if bias is not None:
+        bias = bias.contiguous()
+    idx = idx.contiguous()
+    if idx.dtype != torch.int32 or idx.numel() != 27 * n_out:
+        raise ValueError("idx must be int32 [n_out * 27]")
+    out = torch.empty((n_out, cout), dtype=x.dtype, device=x.device)
+    epi, keep = _epilogue(x, n_out, cout, residual, norm_mod, residual_rows)  # keep: alive until queued
+    L = lib()
+    nbytes = L.spc_conv_products_workspace_bytes(n_in, cout)
+    ws = _workspace(nbytes, x.device)
+    st = L.spc_sparse_conv_products(_stream(x.device), dt, _ptr(x), _ptr(weight.data), _ptr(bias),
+                                    _ptr(out), _ptr(idx), n_out, n_in, cin, cout,
+                                    ctypes.byref(epi), _ptr(ws), nbytes)
+    _check("spc_sparse_conv_products", st)
     return out
 
 

@@ -125,7 +125,8 @@ class SparseResBlock3d(nn.Module):
         (2048 channels over 11,774 instead of 62,710 rows in the SLAT output
         block), conv1 reads them through the fine neighbour table composed
         with up[] (the same values per row and tap, so the same sums, without
-        writing the copies), and conv2 adds the skip from row up[f] in its
+        writing the copies; wide rows as products shared between a coarse
+        row's children, spc_sparse_conv_products), and conv2 adds the skip from row up[f] in its
         epilogue."""
         up = self.updown
         rows = up.fine_rows(x)
@@ -137,17 +138,20 @@ class SparseResBlock3d(nn.Module):
         m = _subm_map(fine)
         c1 = self.conv1.conv
         comp = fine.data.cached("subm3_from_coarse", lambda c: nat.compose_rows(m.token_major, rows))
-        plan = fine.data.cached(("plan", "subm3_from_coarse"), lambda c: nat.conv_plan(
-            comp, ntaps=27, n_out=n_f, n_in=n_c, device=c.device, sections=nat.plan_section(
-                h_c.dtype, ntaps=27, n_out=n_f, cin=_pad32(c1.in_channels),
-                cout=_pad32(c1.out_channels),
-                epi_mode=nat.EPI_NORM_MOD_SILU if self.out_channels in (32, 64, 128) else 0)))
+        nm = None
         if self.out_channels in (32, 64, 128):
-            y1 = self.conv1._conv(h_c, comp, n_f, plan,
-                                  norm_mod=(scale.float(), shift.float(), fine.coords,
-                                            self.norm2.eps))
+            nm = (scale.float(), shift.float(), fine.coords, self.norm2.eps)
+        if self.conv1._use_products(h_c.dtype, n_f, n_c):
+            # the fine rows share their coarse rows' products
+            y1 = self.conv1._conv_products(h_c, comp, n_f, norm_mod=nm)
         else:
-            y1 = self.conv1._conv(h_c, comp, n_f, plan)
+            plan = fine.data.cached(("plan", "subm3_from_coarse"), lambda c: nat.conv_plan(
+                comp, ntaps=27, n_out=n_f, n_in=n_c, device=c.device, sections=nat.plan_section(
+                    h_c.dtype, ntaps=27, n_out=n_f, cin=_pad32(c1.in_channels),
+                    cout=_pad32(c1.out_channels),
+                    epi_mode=nat.EPI_NORM_MOD_SILU if nm else 0)))
+            y1 = self.conv1._conv(h_c, comp, n_f, plan, norm_mod=nm)
+        if nm is None:
             y1 = nat.layernorm_mod_silu(y1, scale.float(), shift.float(), fine.coords,
                                         eps=self.norm2.eps)
         h = fine.replace(y1)

@@ -619,6 +619,40 @@ class _ConvCore:
         return _run(run, feats, c.weight, c.bias)
 
 
+    def _use_products(self, dtype: torch.dtype, n_out: int, n_in: int) -> bool:
+        """Whether a 27-tap conv of n_out rows over n_in source rows forms
+        each (source row, tap) product once (_conv_products).  Measured on
+        shells, 128 output channels, bf16, with the norm epilogue, in us (conv
+        / products), n_out 5.3 n_in: 66,779 rows C_in 2048 1173 / 215, 512
+        324 / 116, 256 183 / 97, 128 113 / 89; 1,512 rows 2048 537 / 51, 256
+        83 / 22.  Without an epilogue C_in 256 gains (131 / 88; 49 / 31 at
+        19,173 rows) and 128 loses (77 / 87; 28.4 / 29.7), so the line is at
+        256.  The dense product multiplies all 27 taps of every source row,
+        the conv ~27 of every output row: below about 3 output rows to a
+        source row the products' F32 traffic is no longer paid for.  Their
+        buffer is held to 1 GiB."""
+        c = self.conv
+        return (dtype in (torch.bfloat16, torch.float16) and self._q8 is None
+                and c.in_channels >= 256 and c.in_channels % 64 == 0 and c.out_channels % 32 == 0
+                and 54 * c.in_channels * c.out_channels < 1 << 31
+                and n_out >= 3 * n_in and 108 * n_in * c.out_channels <= 1 << 30)
+
+    def _conv_products(self, feats: torch.Tensor, idx: torch.Tensor, n_out: int,
+                       norm_mod: Optional[tuple] = None) -> torch.Tensor:
+        c = self.conv
+        if feats.dim() != 2 or feats.shape[1] != c.in_channels:
+            raise ValueError(f"expected feats [N, {c.in_channels}], got {tuple(feats.shape)}")
+        nat._need_gpu(feats)
+
+        def run():
+            x = feats.detach().contiguous()
+            return nat.sparse_conv_products(x, self._weight_operand(x.dtype, x.device),
+                                            self._bias_operand(x.dtype, x.device), idx,
+                                            n_out=n_out, norm_mod=norm_mod)
+
+        return _run(run, feats, c.weight, c.bias)
+
+
 class SparseConv3d(nn.Module, _ConvCore):
     """SparseConv3d(in_channels, out_channels, kernel_size, stride=1,
     dilation=1, padding=None, bias=True, indice_key=None)
