@@ -262,8 +262,9 @@ int spc_sparse_conv(spc_stream_t stream, int dtype, const void* x, int w_dtype, 
                     int64_t n_out, int64_t n_in, int64_t cin, int64_t cout);
 
 /* Tile plan: the per-tile setup of the conv kernel (active tap set,
- * deduplicated source rows, slot table) for both tile geometries (the
- * 256-row tiles, then the small ones; see spc_conv_set_tile_geometry),
+ * deduplicated source rows, slot table) for the tile geometries (the
+ * 256-row tiles, then the small ones, then, for 65,537 to 81,920 rows of 27
+ * taps, the 320-row ones; see spc_conv_set_tile_geometry),
  * built once per index table and reused by every conv over it -- like the
  * map, it depends only on
  * (idx, idx_layout, row_perm, ntaps, n_out, n_in), not on channels or
@@ -276,13 +277,14 @@ size_t spc_conv_plan_bytes(int64_t n_out, int64_t ntaps);
 int spc_conv_plan(spc_stream_t stream, const int32_t* idx, int idx_layout,
                   const int32_t* row_perm, int64_t ntaps, int64_t n_out, int64_t n_in, void* plan,
                   size_t plan_bytes);
-/* spc_conv_plan building only the given sections (SPC_PLAN_WIDE and / or
- * SPC_PLAN_SMALL) of a plan of the same size: a conv whose tile geometry
+/* spc_conv_plan building only the given sections (any of SPC_PLAN_WIDE,
+ * SPC_PLAN_SMALL and SPC_PLAN_LONG) of a plan of the same size: a conv whose tile geometry
  * finds its section unbuilt sets its tiles up itself (same results,
  * slower), so callers that rebuild plans often (per call) build only the
  * geometry their convs run. */
 #define SPC_PLAN_WIDE 1u
 #define SPC_PLAN_SMALL 2u
+#define SPC_PLAN_LONG 4u
 int spc_conv_plan_sections(spc_stream_t stream, const int32_t* idx, int idx_layout,
                            const int32_t* row_perm, int64_t ntaps, int64_t n_out, int64_t n_in,
                            uint32_t sections, void* plan, size_t plan_bytes);
@@ -292,7 +294,7 @@ int spc_sparse_conv_plan(spc_stream_t stream, int dtype, const void* x, int w_dt
                          const void* plan, int64_t ntaps, int64_t n_out, int64_t n_in,
                          int64_t cin, int64_t cout);
 
-/* Tile geometry of the conv kernel.  Every conv runs on one of three:
+/* Tile geometry of the conv kernel.  Every conv runs on one of four:
  *   SPC_TILES_WIDE   256-row tiles over an 895-row double-buffered stage,
  *                    one 8-wave workgroup per CU (long tiles: wide channels);
  *   SPC_TILES_SMALL  128-row tiles (64 for 8 taps) over a 511-row stage,
@@ -303,25 +305,32 @@ int spc_sparse_conv_plan(spc_stream_t stream, int dtype, const void* x, int w_dt
  *                    in four buffers, one 8-wave workgroup per CU);
  *   SPC_TILES_TALL   256-row tiles over a 559-row stage, three 4-wave
  *                    workgroups per CU (one-chunk rows: 16-bit C_in = 32 with
- *                    C_out 32 or 64); reads the wide tiles' plan section.
+ *                    C_out 32 or 64); reads the wide tiles' plan section;
+ *   SPC_TILES_LONG   320-row tiles over a 1119-row double-buffered stage (a
+ *                    tile of up to 1343 rows takes both buffers as one):
+ *                    16-bit convs of C_out 128 that 256-row tiles would
+ *                    leave a nearly empty second round of the CUs.
  * All give the same results.  By default (SPC_TILES_AUTO) each conv picks
  * by shape; spc_conv_set_tile_geometry forces one for every later conv of
  * the process (measurements, tests; initially from the environment
- * variable SPC_CONV_GEOMETRY = "wide" / "small" / "tall").  The small tiles
+ * variable SPC_CONV_GEOMETRY = "wide" / "small" / "tall" / "long").  The small tiles
  * apply to packed weights with 27 or 8 taps, the tall ones to packed
  * weights with 27 taps and C_out a multiple of 32, without the norm
- * epilogue or weight classes (elsewhere a forced geometry that does not
- * apply leaves the choice by shape).  Plans (spc_conv_plan) hold the wide
- * and the small sections.  No reference counterpart. */
+ * epilogue or weight classes, the long ones to packed 16-bit weights with
+ * 27 taps and C_out a multiple of 128 (elsewhere a forced geometry that does not
+ * apply leaves the choice by shape).  Plans (spc_conv_plan) hold the wide,
+ * the small and, for the row counts the long tiles are picked at, the long
+ * section.  No reference counterpart. */
 #define SPC_TILES_AUTO 0
 #define SPC_TILES_WIDE 1
 #define SPC_TILES_SMALL 2
 #define SPC_TILES_TALL 3
+#define SPC_TILES_LONG 4
 int spc_conv_set_tile_geometry(int geometry);
-/* The geometry (SPC_TILES_WIDE / SMALL / TALL) a conv with packed weights
+/* The geometry (SPC_TILES_WIDE / SMALL / TALL / LONG) a conv with packed weights
  * and these arguments runs now (epi_mode a spc_epilogue_mode, class_rows 0
  * without weight classes); SPC_TILES_SMALL reads the small plan section,
- * the others the wide one. */
+ * SPC_TILES_LONG the long one, the others the wide one. */
 int spc_conv_tile_geometry(int dtype, int w_dtype, int64_t ntaps, int64_t n_out, int64_t cin,
                            int64_t cout, int64_t class_rows, int epi_mode);
 

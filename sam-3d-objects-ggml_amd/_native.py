@@ -457,14 +457,14 @@ def convert(x: torch.Tensor, dtype: torch.dtype, out: torch.Tensor | None = None
     return out
 
 
-TILES_AUTO, TILES_WIDE, TILES_SMALL, TILES_TALL = 0, 1, 2, 3
-PLAN_WIDE, PLAN_SMALL = 1, 2
+TILES_AUTO, TILES_WIDE, TILES_SMALL, TILES_TALL, TILES_LONG = 0, 1, 2, 3, 4
+PLAN_WIDE, PLAN_SMALL, PLAN_LONG = 1, 2, 4
 
 
 def tile_geometry(dtype: torch.dtype, *, ntaps: int, n_out: int, cin: int, cout: int,
                   q8: bool = False, class_rows: int = 0, epi_mode: int = 0) -> int:
     """spc_conv_tile_geometry: the geometry (TILES_WIDE / TILES_SMALL /
-    TILES_TALL) a packed-weight conv with these arguments runs now."""
+    TILES_TALL / TILES_LONG) a packed-weight conv with these arguments runs now."""
     dt = dtype_code(dtype)
     return lib().spc_conv_tile_geometry(dt, Q8_0 if q8 else dt, ntaps, n_out, cin, cout,
                                         class_rows, epi_mode)
@@ -472,17 +472,17 @@ def tile_geometry(dtype: torch.dtype, *, ntaps: int, n_out: int, cin: int, cout:
 
 def plan_section(dtype: torch.dtype, *, ntaps: int, n_out: int, cin: int, cout: int,
                  q8: bool = False, class_rows: int = 0, epi_mode: int = 0) -> int:
-    """The plan section (PLAN_WIDE / PLAN_SMALL) a packed-weight conv with
-    these arguments reads: the small tiles read the small section, the wide
-    and the tall tiles the wide one."""
+    """The plan section (PLAN_WIDE / PLAN_SMALL / PLAN_LONG) a packed-weight
+    conv with these arguments reads: the small and the long tiles read their
+    own, the wide and the tall tiles the wide one."""
     g = tile_geometry(dtype, ntaps=ntaps, n_out=n_out, cin=cin, cout=cout, q8=q8,
                       class_rows=class_rows, epi_mode=epi_mode)
-    return PLAN_SMALL if g == TILES_SMALL else PLAN_WIDE
+    return {TILES_SMALL: PLAN_SMALL, TILES_LONG: PLAN_LONG}.get(g, PLAN_WIDE)
 
 
 def set_tile_geometry(geometry: int) -> None:
-    """spc_conv_set_tile_geometry: TILES_WIDE / TILES_SMALL / TILES_TALL
-    force the conv kernel's tile geometry for every later conv of the
+    """spc_conv_set_tile_geometry: TILES_WIDE / TILES_SMALL / TILES_TALL /
+    TILES_LONG force the conv kernel's tile geometry for every later conv of the
     process (where it applies); TILES_AUTO (the default) lets each conv pick
     by shape.  Results are the same."""
     _check("spc_conv_set_tile_geometry", lib().spc_conv_set_tile_geometry(int(geometry)))
@@ -491,7 +491,7 @@ def set_tile_geometry(geometry: int) -> None:
 def conv_plan(idx: torch.Tensor | None, *, ntaps: int, n_out: int, n_in: int | None = None,
               idx_layout: int = IDX_TOKEN_MAJOR,
               row_perm: torch.Tensor | None = None, device=None,
-              sections: int = PLAN_WIDE | PLAN_SMALL) -> torch.Tensor:
+              sections: int = PLAN_WIDE | PLAN_SMALL | PLAN_LONG) -> torch.Tensor:
     """spc_conv_plan_sections: the conv kernel's per-tile setup for this
     index table (reusable by every conv over it), for the tile geometries in
     `sections` (a conv whose geometry finds no plan sets its tiles up)."""

@@ -455,12 +455,13 @@ BridgePlan* bridge_plan(BridgeDev& bd, hipStream_t s, int64_t n, int geometry) {
 }
 
 // Tile-geometry override (spc_conv_set_tile_geometry; initially from
-// SPC_CONV_GEOMETRY=wide / small / tall): 0 = each conv picks by shape.
+// SPC_CONV_GEOMETRY=wide / small / tall / long): 0 = each conv picks by shape.
 std::atomic<int> g_geometry{[] {
     const char* e = getenv("SPC_CONV_GEOMETRY");
     if (e && strcmp(e, "wide") == 0) return SPC_TILES_WIDE;
     if (e && strcmp(e, "small") == 0) return SPC_TILES_SMALL;
     if (e && strcmp(e, "tall") == 0) return SPC_TILES_TALL;
+    if (e && strcmp(e, "long") == 0) return SPC_TILES_LONG;
     return SPC_TILES_AUTO;
 }()};
 int geometry_override() { return g_geometry.load(std::memory_order_relaxed); }
@@ -604,14 +605,15 @@ int spc_convert(spc_stream_t stream, int src_dtype, const void* src, int dst_dty
 
 size_t spc_conv_plan_bytes(int64_t n_out, int64_t ntaps) {
     if (n_out <= 0 || (ntaps != 27 && ntaps != 8 && ntaps != 1)) return 0;
-    return (size_t)(plan_wide_bytes(n_out, (int)ntaps) + plan_small_bytes(n_out, (int)ntaps));
+    return (size_t)(plan_wide_bytes(n_out, (int)ntaps) + plan_small_bytes(n_out, (int)ntaps) +
+                    plan_long_bytes(n_out, (int)ntaps));
 }
 
 int spc_conv_plan(spc_stream_t stream, const int32_t* idx, int idx_layout,
                   const int32_t* row_perm, int64_t ntaps, int64_t n_out, int64_t n_in, void* plan,
                   size_t plan_bytes) {
     return spc_conv_plan_sections(stream, idx, idx_layout, row_perm, ntaps, n_out, n_in,
-                                  SPC_PLAN_WIDE | SPC_PLAN_SMALL, plan, plan_bytes);
+                                  SPC_PLAN_WIDE | SPC_PLAN_SMALL | SPC_PLAN_LONG, plan, plan_bytes);
 }
 
 int spc_conv_plan_sections(spc_stream_t stream, const int32_t* idx, int idx_layout,
@@ -627,7 +629,7 @@ int spc_conv_plan_sections(spc_stream_t stream, const int32_t* idx, int idx_layo
     if (n_out == 0) return SPC_OK;
     if ((!idx && (ntaps != 1 || n_in != n_out)) || !plan || ((uintptr_t)plan & 255u) != 0 ||
         (idx_layout != SPC_IDX_TOKEN_MAJOR && idx_layout != SPC_IDX_OFFSET_MAJOR) ||
-        (sections & ~(SPC_PLAN_WIDE | SPC_PLAN_SMALL)) != 0) {
+        (sections & ~(SPC_PLAN_WIDE | SPC_PLAN_SMALL | SPC_PLAN_LONG)) != 0) {
         set_last_error("spc_conv_plan: null / misaligned (256 bytes) pointer, bad layout or "
                        "unknown section bits");
         return SPC_BAD_ARG;
@@ -643,7 +645,8 @@ int spc_conv_plan_sections(spc_stream_t stream, const int32_t* idx, int idx_layo
     a.n_in = n_in;
     a.idx_layout = idx_layout;
     a.ntaps = (int32_t)ntaps;
-    // the wide tiles' plans, then the small tiles'; a section not asked for
+    // the wide tiles' plans, then the small tiles', then the long tiles' where
+    // the row count has them; a section not asked for
     // has its tiles' markers cleared (its convs set their tiles up themselves)
     char* pl = static_cast<char*>(plan);
     char* ps = pl + plan_wide_bytes(n_out, (int)ntaps);
@@ -661,6 +664,9 @@ int spc_conv_plan_sections(spc_stream_t stream, const int32_t* idx, int idx_layo
     if (ntaps == 27) {
         section(std::integral_constant<int, 27>{}, GeoWide{}, pl, w);
         section(std::integral_constant<int, 27>{}, GeoSmall<27>{}, ps, sm);
+        if (plan_long_bytes(n_out, 27) > 0)
+            section(std::integral_constant<int, 27>{}, GeoLong{}, ps + plan_small_bytes(n_out, 27),
+                    (sections & SPC_PLAN_LONG) != 0);
     } else if (ntaps == 8) {
         section(std::integral_constant<int, 8>{}, GeoWide{}, pl, w);
         section(std::integral_constant<int, 8>{}, GeoSmall<8>{}, ps, sm);
@@ -871,6 +877,7 @@ int spc_conv_tile_geometry(int dtype, int w_dtype, int64_t ntaps, int64_t n_out,
         using T = decltype(t_c);
         constexpr bool Q8 = decltype(q8_c)::value;
         if (ntaps == 27 && use_tall_tiles<T, Q8, true, 27>(a)) g = SPC_TILES_TALL;
+        else if (ntaps == 27 && use_long_tiles<T, Q8, true, 27>(a)) g = SPC_TILES_LONG;
         else if (ntaps == 27 && use_small_tiles<T, Q8, true, 27>(a)) g = SPC_TILES_SMALL;
         else if (ntaps == 8 && use_small_tiles<T, Q8, true, 8>(a)) g = SPC_TILES_SMALL;
     };
@@ -882,7 +889,7 @@ int spc_conv_tile_geometry(int dtype, int w_dtype, int64_t ntaps, int64_t n_out,
 
 int spc_conv_set_tile_geometry(int geometry) {
     if (geometry != SPC_TILES_AUTO && geometry != SPC_TILES_WIDE && geometry != SPC_TILES_SMALL &&
-        geometry != SPC_TILES_TALL) {
+        geometry != SPC_TILES_TALL && geometry != SPC_TILES_LONG) {
         set_last_error("spc_conv_set_tile_geometry: unknown geometry %d", geometry);
         return SPC_BAD_ARG;
     }

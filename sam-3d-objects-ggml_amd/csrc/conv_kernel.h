@@ -259,7 +259,7 @@ constexpr int kWinWords = 1024;  // dedupe bitmap: 32768 source rows
 constexpr int kWinWordsWide = 2048;
 constexpr int kHashBits = 11;    // wider spans: LDS hash of the tile's source rows
 constexpr int kHashSlots = 1 << kHashBits;  // 64-bit slots: row | rank << 32
-constexpr int kSortCap = 1024;   // distinct rows collected after hashing (> any stage's UMAX)
+constexpr int kSortCap = 1472;   // distinct rows collected after hashing (> any stage's UCAP)
 constexpr int kSetupScratchWords = 2 * kWinWordsWide > 2 * kHashSlots + 2 * kSortCap
                                        ? 2 * kWinWordsWide
                                        : 2 * kHashSlots + 2 * kSortCap;
@@ -288,6 +288,12 @@ constexpr int kSegs = 4;        // 16-byte segments per staged 64-byte row chunk
 //             tiles' plans (same row tiles, slot keys and plan layout); a tile
 //             whose union exceeds its stage takes the per-tap fallback, two
 //             taps per round, about four times the staged tile's time.
+//   GeoLong   320 rows, 1119-row stage, otherwise GeoWide: for the row counts
+//             whose 256-row tiles just miss one round of the CUs (65,537 to
+//             81,920 rows of 128 channels).  A shell's 320-row tile references
+//             ~1,000 rows, 1,111 at most over twelve poses of four; one past
+//             the stage (up to 1,343) takes both buffers as one, staged
+//             between its chunks instead of behind them.
 //   GeoQuad   GeoSmall<8>'s 64-row tiles and plan over four 511-row buffers
 //             (128 KB, one workgroup per CU): a tile stages four channel
 //             chunks at once, so a stride-2 conv over 16-bit rows of up to
@@ -315,8 +321,12 @@ struct Geo {
     static constexpr int UMAX = UMAX_;
     static constexpr int NBUF = NBUF_;
     static constexpr bool SW = SW_;
+    static constexpr bool LONG = TM_ == 320;
+    // union rows a tile may have: the long tiles' may exceed a buffer and
+    // take both
+    static constexpr int UCAP = LONG ? PUMAX_ : UMAX_;
     static constexpr int PITCH = SW ? 4 : 5;            // 16-byte units per staged row
-    static constexpr int UROWCAP = (UMAX + 3) / 4 * 4;  // union-row table (16-byte multiple)
+    static constexpr int UROWCAP = (UCAP + 3) / 4 * 4;  // union-row table (16-byte multiple)
     static constexpr int PUROWCAP = (PUMAX_ + 3) / 4 * 4;  // the plan's union-row table
     // the plan section the geometry reads: the 256-row tiles' (up to 895
     // union rows) or the small tiles'
@@ -328,6 +338,14 @@ struct Geo {
     __host__ __device__ static constexpr int key(int r) { return SW ? 4 * r + swz(r) : 5 * r; }
     __host__ __device__ static constexpr int unit(int k, int s) { return SW ? (k ^ s) : k + s; }
     __host__ __device__ static constexpr int seg_pos(int r, int s) { return unit(key(r), s); }
+    // Position of tile row r among a tap's TM slot keys: 64-row groups, row
+    // 16 i + j of a group at 4 j + i; the long tiles' 80-row waves hold such a
+    // group and then its last 16 rows in order.
+    __host__ __device__ static constexpr int slot_pos(int r) {
+        if (!LONG) return (r & ~63) | ((r & 15) << 2) | ((r >> 4) & 3);
+        const int q = r % 80;
+        return r - q + (q < 64 ? ((q & 15) << 2) | (q >> 4) : q);
+    }
     // One row tile's plan: header (U, tap mask, fast flag, tap words),
     // output rows, union rows, slot keys.  It depends only on the index
     // table, its layout, the row order and NTAPS -- not on channels or
@@ -344,6 +362,7 @@ template <int NTAPS>
 using GeoSmall = Geo<NTAPS == 8 ? 64 : 128, 511, 1, true>;
 using GeoTall = Geo<256, 559, 1, true, 895>;
 using GeoQuad = Geo<64, 511, 4, true>;
+using GeoLong = Geo<320, 1119, 2, true, 1343>;
 static_assert(GeoWide::STAGE == 3584 && GeoSmall<27>::STAGE == 2048 && GeoTall::STAGE == 2240,
               "stage geometry");
 static_assert(GeoQuad::plan_tile_bytes(8) == GeoSmall<8>::plan_tile_bytes(8) && !GeoQuad::WIDE_PLAN,
@@ -353,7 +372,9 @@ static_assert(GeoTall::WIDE_PLAN && GeoTall::plan_tile_bytes(27) == GeoWide::pla
               "the tall tiles read the wide plan");
 
 // Plan buffer: the GeoWide plan of every 256-row tile, then the GeoSmall
-// plan of every small tile (a conv picks its geometry by shape).
+// plan of every small tile (a conv picks its geometry by shape), then, for
+// the row counts the long tiles are for, the GeoLong plan of every 320-row
+// tile.
 __host__ __device__ constexpr int64_t plan_wide_bytes(int64_t n_out, int ntaps) {
     return (n_out + GeoWide::TM - 1) / GeoWide::TM * GeoWide::plan_tile_bytes(ntaps);
 }
@@ -362,12 +383,15 @@ __host__ __device__ constexpr int64_t plan_small_bytes(int64_t n_out, int ntaps)
                       : (n_out + 127) / 128 * GeoSmall<27>::plan_tile_bytes(ntaps);
 }
 
+// (256 workgroups are a round of the MI355X)
+__host__ __device__ constexpr int64_t plan_long_bytes(int64_t n_out, int ntaps) {
+    return ntaps == 27 && n_out > 256 * GeoWide::TM && n_out <= 256 * GeoLong::TM
+               ? (n_out + GeoLong::TM - 1) / GeoLong::TM * GeoLong::plan_tile_bytes(27)
+               : 0;
+}
+
 constexpr int kTapWords = 8;  // step taps, four per word: up to 28 steps per chunk
 constexpr int32_t kPlanMagic = 0x314e4c50;  // header word 3 of every built plan tile
-
-// Position of tile row r among a tap's TM slot keys: 64-row groups, row
-// 16 i + j of a group at 4 j + i.
-__host__ __device__ constexpr int slot_pos(int r) { return (r & ~63) | ((r & 15) << 2) | ((r >> 4) & 3); }
 
 // Shared-memory arrays of one tile's setup.
 struct TileLds {
@@ -394,7 +418,7 @@ struct TileLds {
 template <int NTAPS, int NT, int PD, typename GEO>
 __device__ __forceinline__ void tile_setup(const ConvArgs& a, int64_t r0, const TileLds& L) {
     constexpr int TM = GEO::TM;
-    constexpr int kUMax = GEO::UMAX;
+    constexpr int kUMax = GEO::UCAP;
     constexpr int NW = NT / 64;
     constexpr int NQ = NTAPS * TM;
     constexpr int EPT = (NQ + NT - 1) / NT;
@@ -649,7 +673,7 @@ __device__ __forceinline__ void tile_setup(const ConvArgs& a, int64_t r0, const 
         for (int q = tid; q < NQ; q += NT) {
             const int o = q / TM;
             const int r = q - o * TM;
-            L.sidx[o * TM + slot_pos(r)] = stg[r * NTAPS + o];
+            L.sidx[o * TM + GEO::slot_pos(r)] = stg[r * NTAPS + o];
         }
     }
     if (tid == 0) {
@@ -760,7 +784,15 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
     __shared__ u32x4 Au[NBUF * STAGE];  // A buffers: (U + 1) rows x 64 bytes each
     __shared__ __attribute__((aligned(16))) uint16_t sidx[NQ + TM];  // slot keys; row NTAPS = zeros
     __shared__ __attribute__((aligned(16))) uint32_t tlw[kTapWords]; // step taps, 4 per word
-    __shared__ __attribute__((aligned(16))) int32_t urow[GEO::UROWCAP];  // source row of each union slot
+    // source row of each union slot.  The long tiles' lie at the end of the A
+    // area: they are read before the first chunk's barrier, the second buffer
+    // is filled after it, and a tile taking both buffers ends short of them.
+    __shared__ __attribute__((aligned(16))) int32_t urow_own[GEO::LONG ? 4 : GEO::UROWCAP];
+    int32_t* const urow = GEO::LONG ? reinterpret_cast<int32_t*>(Au + NBUF * STAGE) - GEO::UROWCAP : urow_own;
+    static_assert(!GEO::LONG || ((GEO::UCAP + 1) * 4 + 63) / 64 * 64 + GEO::UROWCAP / 4 <= NBUF * STAGE,
+                  "the union rows lie past a tile taking both buffers");
+    static_assert(!GEO::LONG || kSetupScratchWords * 4 + GEO::UROWCAP * 4 <= ABYTES,
+                  "the union rows lie past the setup scratch");
     __shared__ __attribute__((aligned(16))) int32_t srow[TM];        // output row of each tile row
     __shared__ int32_t wsum[NW];
     __shared__ __attribute__((aligned(16))) int32_t misc[8];
@@ -880,7 +912,7 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
             for (int r = tid; r < TM; r += NT) {
                 srow[r] = r < nr ? (int32_t)(r0 + r) : -1;
                 urow[r] = (int32_t)(r0 + r);
-                sidx[slot_pos(r)] = (uint16_t)GEO::key(r < nr ? r : nr);
+                sidx[GEO::slot_pos(r)] = (uint16_t)GEO::key(r < nr ? r : nr);
                 sidx[TM + r] = (uint16_t)GEO::key(nr);
             }
             if (tid < kTapWords) tlw[tid] = tid == 0 ? 0xffffff00u : 0xffffffffu;  // tap 0, then padding
@@ -1118,6 +1150,12 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
                 for (int i = 0; i < 4 && 4 * q + i < FA; ++i)
                     sl[4 * q + i] = (int)((i & 1) ? v[i >> 1] >> 16 : v[i >> 1] & 0xffffu);
             }
+        } else if constexpr (BR == 16 && WTM == 80) {
+            const u32x2 v = *reinterpret_cast<const u32x2*>(st + wm * WTM + 4 * (lane & 15));
+#pragma unroll
+            for (int i = 0; i < 4 && i < FA; ++i)
+                sl[i] = (int)((i & 1) ? v[i >> 1] >> 16 : v[i >> 1] & 0xffffu);
+            if constexpr (FA > 4) sl[4] = st[wm * WTM + 64 + (lane & 15)];
         } else if constexpr (BR == 16 && WTM == 32) {
             const uint32_t v = *reinterpret_cast<const uint32_t*>(
                 st + (wm * WTM & ~63) + 4 * (lane & 15) + ((wm * WTM >> 4) & 3));
@@ -1125,7 +1163,7 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
             if constexpr (FA > 1) sl[1] = (int)(v >> 16);
         } else {
 #pragma unroll
-            for (int i = 0; i < FA; ++i) sl[i] = st[slot_pos(wm * WTM + i * BR + (lane % BR))];
+            for (int i = 0; i < FA; ++i) sl[i] = st[GEO::slot_pos(wm * WTM + i * BR + (lane % BR))];
         }
     };
     const auto fm_all = std::integral_constant<int, FM>{};
@@ -1133,7 +1171,7 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
     // The fast path stages through LDS DMA with 32-bit offsets from the
     // tile's lowest source row.
     const int64_t rowbytes = (int64_t)a.cin * ES;
-    const bool dma = fast && nt > 0 && U > 0 && U <= GEO::UMAX &&
+    const bool dma = fast && nt > 0 && U > 0 && U <= GEO::UCAP &&
                      (int64_t)(urow[U - 1] - urow[0] + 1) * rowbytes <= 0x7fffffffLL;
 
     if (dma) {
@@ -1156,10 +1194,13 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
         const uint32_t au_lds = __builtin_amdgcn_readfirstlane(
             (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) u32x4*)Au));
         const int nblk = ((U + 1) * GEO::PITCH + 63) / 64;
+        // a long tile past one buffer takes both, its chunks staged one by one
+        const bool single = GEO::LONG && U > GEO::UMAX;
         // Wave w fills blocks w + NW j.  The per-lane source offsets do not
         // depend on the chunk (it enters as the scalar offset), so they are
         // computed once per tile and kept in registers.
-        constexpr int NJ = (STAGE / 64 + NW - 1) / NW;  // blocks per wave, at most
+        constexpr int NBLK = GEO::LONG ? ((GEO::UCAP + 1) * GEO::PITCH + 63) / 64 : STAGE / 64;
+        constexpr int NJ = (NBLK + NW - 1) / NW;  // blocks per wave, at most
         uint32_t doff[NJ];
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
@@ -1204,7 +1245,12 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
         // it is needed only in its own chunk.  Chunks 0 and 1 are staged
         // together; chunk 0 alone is waited for.
         constexpr bool DR = NBUF == 4 && NTAPS <= 2 * PD && PACKED;
-        constexpr int RS = DR ? 2 * PD : PD;  // weight ring slots
+        // weights are loaded LA steps ahead: a whole group, or two steps where a
+        // step is 20 MFMAs a wave (the long tiles: four would spill, and a
+        // reload behind the prefetches waits for them all)
+        constexpr int LA = GEO::LONG ? 2 : PD;
+        constexpr int RS = DR ? 2 * PD : LA;  // weight ring slots
+        static_assert(PD % LA == 0 && (!DR || LA == PD), "ring geometry");
         static_assert(!DR || (2 * PD * LPS < 64 && NJ < 64), "vmcnt range");
         const int njw = wave < nblk ? min(NJ, (nblk - wave + NW - 1) / NW) : 0;  // this wave's blocks per chunk
         auto stage_chunk = [&](int kc) __attribute__((always_inline)) {
@@ -1215,7 +1261,7 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
         // multiple of PD with steps that read the zero slot (row NTAPS)
         // against the first tap's weights.  A group of PD steps is unrolled;
         // every register-array index inside it is a compile-time constant:
-        // B operands of step i live in ring[i % PD] (loaded PD steps ahead;
+        // B operands of step i live in ring[i % LA] (loaded LA steps ahead;
         // the whole-chunk ring: ring[i], loaded a chunk ahead),
         // A fragments in afr[i % 2] (read one step ahead, within a chunk),
         // union slots in sreg[i % 2] (read two steps ahead; slots do not
@@ -1256,8 +1302,9 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
                 for (int h = 0; h < NPART; ++h) stage_part_rt(0, 0, h);
                 dma_barrier<0>();
                 for (int kc = 0; kc + 1 < kch; ++kc) {
-                    if constexpr (NBUF == 1) lds_barrier();  // the buffer is free
-                    for (int h = 0; h < NPART; ++h) stage_part_rt(kc + 1, NBUF == 1 ? 0 : (kc & 1) ^ 1, h);
+                    if (NBUF == 1 || single) lds_barrier();  // the buffer is free
+                    for (int h = 0; h < NPART; ++h)
+                        stage_part_rt(kc + 1, NBUF == 1 || single ? 0 : (kc & 1) ^ 1, h);
                     dma_barrier<0>();
                 }
             }
@@ -1277,7 +1324,7 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
             {
                 const uint32_t w0 = tw_first[0];
 #pragma unroll
-                for (int p = 0; p < PD; ++p) load_b(b_tap(w0, p), 0, ring[p]);
+                for (int p = 0; p < LA; ++p) load_b(b_tap(w0, p), 0, ring[p]);
                 if constexpr (DR) {
                     const uint32_t w1f = tw_first[1];
 #pragma unroll
@@ -1302,9 +1349,9 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
             }
 
             for (int kc = 0; kc < kch; ++kc) {
-                const int buf = NBUF == 1 ? 0 : NBUF == 2 ? kc & 1 : kc % NBUF;
+                const int buf = NBUF == 1 || single ? 0 : NBUF == 2 ? kc & 1 : kc % NBUF;
                 // two buffers: the next chunk is staged while this one runs
-                const bool more = NBUF == 2 && kc + 1 < kch;
+                const bool more = NBUF == 2 && kc + 1 < kch && !single;
                 if (kc > 0) {
                     if constexpr (DR) {
                         // this chunk has landed: younger than its staging are
@@ -1321,7 +1368,7 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
                             stage_group(kc);
                             dma_barrier<0>();
                         }
-                    } else if constexpr (NBUF == 1) {
+                    } else if (NBUF == 1 || single) {
                         // one buffer: once every wave is done reading the last
                         // chunk (the barrier's fence waits for this wave's LDS
                         // reads), stage this one and wait for it; the weight
@@ -1363,11 +1410,12 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
                         // are re-read behind the barrier, so this read is unused
                         read_frags(buf, sreg[(u + 1) & 1], afr[(u + 1) & 1], fa_const);
                         if constexpr (last_g && (u > 0 || DR)) {
-                            if (u < nreal) mma_step(afr[u & 1], ring[RB + u], fa_const);
+                            if (u < nreal) mma_step(afr[u & 1], ring[RB + u % LA], fa_const);
                         } else {
-                            mma_step(afr[u & 1], ring[RB + u], fa_const);
+                            mma_step(afr[u & 1], ring[RB + u % LA], fa_const);
                         }
-                        load_b(b_tap(wl, u), kc_b, ring[RB + u]);
+                        if constexpr (u + LA < PD) load_b(b_tap(w0, u + LA), kc, ring[u % LA]);
+                        else load_b(b_tap(wl, (u + LA) % PD), kc_b, ring[RB + u % LA]);
                         // issue order: slot reads, then MFMAs interleaved with the
                         // fragment reads and their address arithmetic, then the
                         // weight loads
@@ -1505,7 +1553,7 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
         static_assert(RPN * FP * 4 <= ABYTES && RPN % 32 == 0, "f32 output tile fits the A stage");
         constexpr int G = TN / 4;            // lanes per row
         constexpr int RW = 64 / G;           // rows per wave at a time
-        constexpr int RB = 4;                // row groups in flight per lane
+        constexpr int RB = RPN / (NW * RW) % 4 == 0 ? 4 : 5;  // row groups in flight per lane
         static_assert(RPN % (NW * RW * RB) == 0, "norm epilogue geometry");
         float* of = reinterpret_cast<float*>(Au);
         const int gl = lane % G;
@@ -1777,9 +1825,19 @@ hipError_t launch_conv(hipStream_t s, ConvArgs a) {
     if (grid == 0) return hipSuccess;
     if (a.epi_mode == SPC_EPI_NORM_MOD_SILU && !norm_epilogue_fits<GEO, TN>())
         return hipErrorInvalidValue;  // the tile cannot hold the epilogue's rows
-    // the plan buffer holds the wide plans, then the small ones
-    if (a.plan && !GEO::WIDE_PLAN)
+    // the plan buffer holds the wide plans, then the small ones, then the long ones
+    if (a.plan && GEO::LONG) {
+        const bool has = plan_long_bytes(a.n_out, NTAPS) > 0;
+        a.plan = has ? static_cast<const char*>(a.plan) + plan_wide_bytes(a.n_out, NTAPS) +
+                           plan_small_bytes(a.n_out, NTAPS)
+                     : nullptr;
+        if (!has) {  // nothing to refresh either
+            a.plan_dirty = nullptr;
+            a.idx_cache = nullptr;
+        }
+    } else if (a.plan && !GEO::WIDE_PLAN) {
         a.plan = static_cast<const char*>(a.plan) + plan_wide_bytes(a.n_out, NTAPS);
+    }
     conv_kernel<T, Q8, PACKED, NTAPS, TN, WM, WN, 4, GEO><<<(unsigned)grid, WM * WN * 64, 0, s>>>(a);
     return hipGetLastError();
 }
@@ -1891,6 +1949,26 @@ bool use_tall_tiles(const ConvArgs& a) {
     }
 }
 
+// Long tiles (GeoLong: 320 rows): 16-bit SubM convs of 128 output channels
+// whose 256-row tiles need a second round of the CUs that the 320-row ones
+// do not -- otherwise a round for the last few tiles.  66,779 rows C 128, bf16:
+// 73.8 -> 57.4 us (small tiles before), with the norm epilogue 113 -> 71.5
+// (wide tiles in two rounds); 79,659 rows 71.3 -> 56.6; C_in 256, 131 -> 94.
+// Forced (SPC_TILES_LONG), any packed 16-bit 27-tap conv whose C_out is a
+// multiple of 128, except Q8_0 and weight classes.
+template <typename T, bool Q8, bool PACKED, int NTAPS>
+bool use_long_tiles(const ConvArgs& a) {
+    if constexpr (!PACKED || Q8 || NTAPS != 27 || sizeof(T) != 2) {
+        return false;
+    } else {
+        if (a.class_rows > 0 || a.cout % 128 != 0) return false;
+        if (a.epi_mode == SPC_EPI_NORM_MOD_SILU && a.cout != 128) return false;
+        if (a.geometry != SPC_TILES_AUTO) return a.geometry == SPC_TILES_LONG;
+        return a.cout == 128 && ceil_div(a.n_out, GeoWide::TM) > a.num_cu &&
+               ceil_div(a.n_out, GeoLong::TM) <= a.num_cu;
+    }
+}
+
 template <typename T, bool Q8, bool PACKED, int NTAPS>
 hipError_t dispatch_tall(hipStream_t s, const ConvArgs& a) {
     return launch_conv<T, Q8, PACKED, NTAPS, 32, 4, 1, GeoTall>(s, a);
@@ -1908,6 +1986,9 @@ hipError_t dispatch_tn(hipStream_t s, const ConvArgs& a) {
     if constexpr (PACKED && NTAPS != 1) {
         if constexpr (NTAPS == 27)
             if (use_tall_tiles<T, Q8, PACKED, NTAPS>(a)) return dispatch_tall<T, Q8, PACKED, NTAPS>(s, a);
+        if constexpr (!Q8 && NTAPS == 27 && sizeof(T) == 2)
+            if (use_long_tiles<T, Q8, PACKED, NTAPS>(a))
+                return launch_conv<T, Q8, PACKED, NTAPS, 128, 4, 2, GeoLong>(s, a);
         if (use_small_tiles<T, Q8, PACKED, NTAPS>(a)) return dispatch_small<T, Q8, PACKED, NTAPS>(s, a);
     }
     const int64_t tiles_m = ceil_div(a.n_out, GeoWide::TM);

@@ -481,3 +481,98 @@ def test_dedupe_paths(spc, orc, dev, geo, dims, path):
                           w_dtype=oracle.BF16, b_dtype=oracle.BF16, nthreads=oracle_threads(),
                           blocked=True)
     check_16bit(f"dedupe via the {path}", from_dev(wp), ref)
+
+
+@pytest.mark.parametrize("dt,cin,cout,last", [
+    ("bf16", 128, 128, 133), ("bf16", 32, 128, 1), ("bf16", 64, 256, 320), ("f16", 96, 128, 16),
+    ("f16", 160, 128, 81)])
+def test_long_tiles_equal_wide(spc, dev, geo, dt, cin, cout, last):
+    """The 320-row tiles against the wide ones, value for value, over a table
+    whose tiles reference 1 to 3,000 source rows: in one buffer (at most
+    1,119), past it in both (1,120 to 1,343) and past both (the per-tap
+    fallback); last tiles of 1 to 320 rows, odd and even chunk counts; plain,
+    residual and norm epilogues, set up in the kernel."""
+    import torch
+
+    nat = geo
+    td = torch.bfloat16 if dt == "bf16" else torch.float16
+    g = torch.Generator(device="cuda").manual_seed(1)
+    widths = [1, 600, 1119, 1120, 1200, 1343, 1344, 3000, 1300, 900]
+    n = 320 * (len(widths) - 1) + last
+    print(f"[case] long tiles {dt} N={n} {cin}->{cout}", flush=True)
+    rows = []
+    for i, wd in enumerate(widths):
+        k = 320 if i + 1 < len(widths) else last
+        lo = min(max(0, 320 * i - 400), n - wd)
+        t = torch.randint(lo, lo + wd, (k, 27), generator=g, device=dev, dtype=torch.int32)
+        if wd in (1119, 1120, 1343, 1344):  # exactly that many distinct rows
+            t.view(-1)[:wd] = torch.arange(lo, lo + wd, device=dev, dtype=torch.int32)
+        else:
+            t[torch.rand((k, 27), generator=g, device=dev) < 0.2] = n  # missing taps
+        rows.append(t)
+    idx = torch.cat(rows).contiguous()
+    unions = [int(torch.unique(r[r < n]).numel()) for r in idx.split(320)]
+    assert {1119, 1120, 1343, 1344} <= set(unions) and max(unions) > 2000
+    coords = torch.zeros((n, 4), dtype=torch.int32, device=dev)
+    coords[n // 2:, 0] = 1
+    r = lambda *s, std=1.0: (torch.randn(s, generator=g, device=dev) * std).to(td)  # noqa: E731
+    x, w, b, res = r(n, cin), r(cout, 27, cin, std=0.03), r(cout), r(n, cout)
+    pw = nat.pack_weights(w)
+    epis = [{}, {"residual": res}]
+    if cout == 128:
+        epis.append({"norm_mod": (r(2, cout), r(2, cout), coords, 1e-6)})
+    for e in epis:
+        nat.set_tile_geometry(nat.TILES_WIDE)
+        yw = nat.sparse_conv(x, pw, b, idx.view(-1), ntaps=27, n_out=n, **e)
+        nat.set_tile_geometry(nat.TILES_LONG)
+        assert nat.tile_geometry(td, ntaps=27, n_out=n, cin=cin, cout=cout) == nat.TILES_LONG
+        yl = nat.sparse_conv(x, pw, b, idx.view(-1), ntaps=27, n_out=n, **e)
+        torch.cuda.synchronize()
+        assert torch.equal(yw, yl), list(e)
+
+
+@pytest.mark.parametrize("n,cout,epi,want", [
+    (65536, 128, 0, "WIDE"), (65537, 128, 0, "LONG"), (81920, 128, 0, "LONG"),
+    (81921, 128, 0, "SMALL"), (66000, 64, 0, "WIDE"), (66000, 128, 2, "LONG"),
+    (40000, 256, 0, "SMALL")])
+def test_long_tiles_are_picked_for_one_round(spc, dev, geo, n, cout, epi, want):
+    import torch
+
+    nat = geo
+    assert nat.tile_geometry(torch.bfloat16, ntaps=27, n_out=n, cin=128, cout=cout,
+                             epi_mode=epi) == getattr(nat, "TILES_" + want)
+    assert nat.tile_geometry(torch.float32, ntaps=27, n_out=n, cin=128, cout=cout) != nat.TILES_LONG
+
+
+def test_long_tiles_planned(spc, dev, geo):
+    """A planned long conv (65,537+ rows), all sections and its own alone,
+    against the wide tiles; and the spconv bridge's self-refreshing plan at
+    that size, over two index tables in turn."""
+    import torch
+
+    nat = geo
+    c = spc.workloads.ellipsoid_batch(4)
+    extra = c[c[:, 0] == 0].copy()
+    extra[:, 0] = 4
+    coords = torch.from_numpy(np.concatenate([c, extra])[:66000]).to(dev)
+    n = coords.shape[0]
+    print(f"[case] long tiles planned N={n}", flush=True)
+    assert n == 66000
+    m = nat.map_build(coords)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    r = lambda *s, std=1.0: (torch.randn(s, generator=g, device=dev) * std).half()  # noqa: E731
+    x, w, b = r(n, 128), r(128, 27, 128, std=0.02), r(128)
+    pw = nat.pack_weights(w)
+    run = lambda p: nat.sparse_conv(x, pw, b, m.token_major, ntaps=27, n_out=n, plan=p)  # noqa: E731
+    nat.set_tile_geometry(nat.TILES_WIDE)
+    yw = run(None)
+    nat.set_tile_geometry(nat.TILES_AUTO)
+    assert nat.plan_section(torch.float16, ntaps=27, n_out=n, cin=128, cout=128) == nat.PLAN_LONG
+    for s in (nat.PLAN_WIDE | nat.PLAN_SMALL | nat.PLAN_LONG, nat.PLAN_LONG, nat.PLAN_WIDE):
+        assert torch.equal(run(nat.conv_plan(m.token_major, ntaps=27, n_out=n, sections=s)), yw)
+    shifted = torch.roll(m.offset_major.view(27, n), 64, 1).contiguous().view(-1)
+    for idx in (m.offset_major, m.offset_major, shifted, m.offset_major):
+        y, msg = nat.spconv_f16_forward(x, w, b, idx, m.mask_sorted, m.argsort)
+        assert msg == ""
+        ref = nat.sparse_conv(x, pw, b, idx, ntaps=27, n_out=n, idx_layout=nat.IDX_OFFSET_MAJOR)
+        assert torch.equal(y, ref)
