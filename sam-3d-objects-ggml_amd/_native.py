@@ -477,6 +477,11 @@ def plan_section(dtype: torch.dtype, *, ntaps: int, n_out: int, cin: int, cout: 
     own, the wide and the tall tiles the wide one."""
     g = tile_geometry(dtype, ntaps=ntaps, n_out=n_out, cin=cin, cout=cout, q8=q8,
                       class_rows=class_rows, epi_mode=epi_mode)
+    return geometry_section(g)
+
+
+def geometry_section(g: int) -> int:
+    """The plan section that tile geometry g reads."""
     return {TILES_SMALL: PLAN_SMALL, TILES_LONG: PLAN_LONG}.get(g, PLAN_WIDE)
 
 

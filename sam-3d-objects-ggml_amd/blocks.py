@@ -254,13 +254,22 @@ class SparseSubdivideBlock3d(nn.Module):
         cm = nat.subdivide_neighbors(pm, n_par)
         c1, c2 = conv1.conv, conv2.conv
         dt = x.feats.dtype
-        # the plans are rebuilt per call: only the tile geometry each conv runs
+        # the plans are rebuilt per call: only the tile geometry each conv runs,
+        # and none for small tiles of all the columns (96 or 192), which each
+        # read it once and set up in the kernel behind each other's loops
+        # (1,227,072 rows 96 -> 96: plan + conv 661 us, conv alone 626)
+        def plan(idx, cout, **shape):
+            g = nat.tile_geometry(dt, ntaps=shape["ntaps"], n_out=shape["n_out"], cin=shape.pop("cin"),
+                                  cout=cout, class_rows=shape.pop("class_rows", 0),
+                                  epi_mode=shape.pop("epi_mode", 0))
+            if g == nat.TILES_SMALL and cout in (96, 192):
+                return None
+            return nat.conv_plan(idx, sections=nat.geometry_section(g), **shape)
+
         if self.merged_taps and c1.in_channels % 32 == 0 and c1.out_channels % 32 == 0:
             idx8, perm, crows = nat.subdivide_tap_classes(pm, n_par)
-            plan8 = nat.conv_plan(idx8, ntaps=8, n_out=8 * crows, n_in=n_par, row_perm=perm,
-                                  sections=nat.plan_section(
-                                      dt, ntaps=8, n_out=8 * crows, cin=c1.in_channels,
-                                      cout=c1.out_channels, class_rows=crows))
+            plan8 = plan(idx8, c1.out_channels, ntaps=8, n_out=8 * crows, n_in=n_par, row_perm=perm,
+                         cin=c1.in_channels, class_rows=crows)
             hp = h_par.detach()
             y1 = _run(lambda: nat.sparse_conv(
                 hp, self._merged_weights(hp.dtype, hp.device), conv1._bias_operand(hp.dtype, hp.device),
@@ -268,17 +277,14 @@ class SparseSubdivideBlock3d(nn.Module):
                 n_classes=8)[:nc], h_par, c1.weight, c1.bias)
         else:
             composed = nat.compose_rows(cm.token_major, parent)
-            plan1 = nat.conv_plan(composed, ntaps=27, n_out=nc, n_in=n_par,
-                                  sections=nat.plan_section(dt, ntaps=27, n_out=nc,
-                                                            cin=_pad32(c1.in_channels),
-                                                            cout=_pad32(c1.out_channels)))
+            plan1 = plan(composed, _pad32(c1.out_channels), ntaps=27, n_out=nc, n_in=n_par,
+                         cin=_pad32(c1.in_channels))
             y1 = conv1._conv(h_par, composed, nc, plan1)
         h = self.sub.assemble(x, coords, y1)
         h.data.cached("subm3", lambda c: cm)  # conv2's map: the same child coordinates
-        h.data.cached(("plan", "subm3"), lambda c: nat.conv_plan(
-            cm.token_major, ntaps=27, n_out=nc, device=c.device, sections=nat.plan_section(
-                dt, ntaps=27, n_out=nc, cin=_pad32(c2.in_channels), cout=_pad32(c2.out_channels),
-                epi_mode=nat.EPI_RESIDUAL)))
+        plan2 = plan(cm.token_major, _pad32(c2.out_channels), ntaps=27, n_out=nc,
+                     cin=_pad32(c2.in_channels), epi_mode=nat.EPI_RESIDUAL)
+        h.data.cached(("plan", "subm3"), lambda c: plan2)
         h = h.replace(nat.group_norm_silu(h.feats, 8 * offs, gn1.num_groups, gn1.weight, gn1.bias,
                                           gn1.eps, silu=True, max_rows=8 * rows_max))
         # the skip on the parent rows (a 1x1x1 conv is row-wise), added to
@@ -286,5 +292,9 @@ class SparseSubdivideBlock3d(nn.Module):
         skip = x.feats if isinstance(self.skip_connection, nn.Identity) \
             else self.skip_connection(x).feats
         if self.out_channels % 32 == 0:
-            return conv2.forward_fused(h, residual=skip, residual_rows=parent)
-        return conv2(h) + h.replace(nat.gather_rows(skip, parent))
+            y = conv2.forward_fused(h, residual=skip, residual_rows=parent)
+        else:
+            y = conv2(h) + h.replace(nat.gather_rows(skip, parent))
+        if plan2 is None:  # later convs over these rows build their own
+            y.data.indice_dict.pop(("plan", "subm3"), None)
+        return y

@@ -879,7 +879,8 @@ int spc_conv_tile_geometry(int dtype, int w_dtype, int64_t ntaps, int64_t n_out,
         if (ntaps == 27 && use_tall_tiles<T, Q8, true, 27>(a)) g = SPC_TILES_TALL;
         else if (ntaps == 27 && use_long_tiles<T, Q8, true, 27>(a)) g = SPC_TILES_LONG;
         else if (ntaps == 27 && use_small_tiles<T, Q8, true, 27>(a)) g = SPC_TILES_SMALL;
-        else if (ntaps == 8 && use_small_tiles<T, Q8, true, 8>(a)) g = SPC_TILES_SMALL;
+        else if (ntaps == 8 && (use_class_tiles<T, Q8, true, 8>(a) || use_small_tiles<T, Q8, true, 8>(a)))
+            g = SPC_TILES_SMALL;
     };
     if (w_dtype == SPC_Q8_0) pick(__bf16{}, std::true_type{});
     else if (dtype == SPC_F32) pick(float{}, std::false_type{});

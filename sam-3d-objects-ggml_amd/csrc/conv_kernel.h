@@ -362,6 +362,7 @@ template <int NTAPS>
 using GeoSmall = Geo<NTAPS == 8 ? 64 : 128, 511, 1, true>;
 using GeoTall = Geo<256, 559, 1, true, 895>;
 using GeoQuad = Geo<64, 511, 4, true>;
+using GeoClass = Geo<128, 511, 1, true>;  // GeoSmall<27>'s tile for the 8-tap weight classes
 using GeoLong = Geo<320, 1119, 2, true, 1343>;
 static_assert(GeoWide::STAGE == 3584 && GeoSmall<27>::STAGE == 2048 && GeoTall::STAGE == 2240,
               "stage geometry");
@@ -1245,10 +1246,10 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
         // it is needed only in its own chunk.  Chunks 0 and 1 are staged
         // together; chunk 0 alone is waited for.
         constexpr bool DR = NBUF == 4 && NTAPS <= 2 * PD && PACKED;
-        // weights are loaded LA steps ahead: a whole group, or two steps where a
-        // step is 20 MFMAs a wave (the long tiles: four would spill, and a
-        // reload behind the prefetches waits for them all)
-        constexpr int LA = GEO::LONG ? 2 : PD;
+        // weights are loaded LA steps ahead: a whole group, or two steps where
+        // four would spill (a reload behind the prefetches waits for them all):
+        // the long tiles' 20 MFMAs a step, the small tiles of 96 and 192 columns
+        constexpr int LA = GEO::LONG || (NBUF == 1 && (TN == 192 || TN == 96)) ? 2 : PD;
         constexpr int RS = DR ? 2 * PD : LA;  // weight ring slots
         static_assert(PD % LA == 0 && (!DR || LA == PD), "ring geometry");
         static_assert(!DR || (2 * PD * LPS < 64 && NJ < 64), "vmcnt range");
@@ -1826,6 +1827,7 @@ hipError_t launch_conv(hipStream_t s, ConvArgs a) {
     if (a.epi_mode == SPC_EPI_NORM_MOD_SILU && !norm_epilogue_fits<GEO, TN>())
         return hipErrorInvalidValue;  // the tile cannot hold the epilogue's rows
     // the plan buffer holds the wide plans, then the small ones, then the long ones
+    if (NTAPS == 8 && GEO::TM == 128) a.plan = nullptr;  // the class tiles have no plan section
     if (a.plan && GEO::LONG) {
         const bool has = plan_long_bytes(a.n_out, NTAPS) > 0;
         a.plan = has ? static_cast<const char*>(a.plan) + plan_wide_bytes(a.n_out, NTAPS) +
@@ -1885,6 +1887,12 @@ hipError_t dispatch_small(hipStream_t s, const ConvArgs& a) {
         if constexpr (Q8 && G::TM == 128) return launch_conv<T, Q8, PACKED, NTAPS, 128, 1, 4, G>(s, a);
         else return launch_conv<T, Q8, PACKED, NTAPS, 128, 2, 2, G>(s, a);
     }
+    // 192 columns in two workgroups a CU, 96 in three (weights two steps ahead:
+    // four would spill at their register budgets)
+    if constexpr (!Q8 && PACKED && sizeof(T) == 2 && G::TM == 128) {
+        if (a.cout % 192 == 0 && a.cout % 128 != 0) return launch_conv<T, Q8, PACKED, NTAPS, 192, 2, 2, G>(s, a);
+        if (a.cout % 96 == 0 && a.cout % 64 != 0) return launch_conv<T, Q8, PACKED, NTAPS, 96, 2, 2, G>(s, a);
+    }
     if (tn == 64) return launch_conv<T, Q8, PACKED, NTAPS, 64, 2, 2, G>(s, a);
     if constexpr (G::TM == 128) return launch_conv<T, Q8, PACKED, NTAPS, 32, 4, 1, G>(s, a);
     else return launch_conv<T, Q8, PACKED, NTAPS, 32, 2, 1, G>(s, a);
@@ -1901,16 +1909,49 @@ hipError_t dispatch_small(hipStream_t s, const ConvArgs& a) {
 //     f32) into at most 64 output channels, where a wide tile is mostly
 //     setup and staging latency (the mesh levels: 31.8 -> 23.3 us at 128^3
 //     C=64, 50.8 -> 38.7 us at 256^3 C=32);
-//   - 128-column tiles that need more than one round of the CUs, so the
-//     workgroups sharing a CU drift apart (SubM 1024 -> 1024 over 11,774
-//     rows: 627 -> 572 us; 128 -> 1024: 105 -> 89 us).
+//   - 128-, 192- and 96-column tiles by the rounds of the CUs they need (the
+//     rules below), where the workgroups sharing a CU drift apart.
 // A single round of long wide tiles stays wide: the double-buffered stage
 // overlaps every chunk's staging with the MFMAs, which the small tiles'
 // synchronised workgroups cannot (C=128 over 62,710 rows: 57 vs 104 us;
 // f32 C=64 over 21,766 rows: 62.9 vs 65.2 us).
 // Packed weights, 27 or 8 taps (the dense 1 x 1 x 1 conv keeps the wide
-// tiles, as do weight classes, the 96- / 192-column tiles and the norm
+// tiles, as do weight classes other than the class tiles' and the norm
 // epilogue over 128 channels).
+// For 16-bit weights the 128-, 192- and 96-column tiles choose by what the last
+// round of the CUs holds (t: tiles of 256 rows; us, wide / small):
+//   128  two small workgroups a CU run half rounds, so they gain while the last
+//        wide round is at most half full, and lose the wide tiles' overlapped
+//        staging where it is fuller: 1024 -> 1024 at t / CUs 1.06 501 / 449,
+//        1.47 577 / 530, 1.62 605 / 643, 1.91 640 / 676, 2.41 926 / 849,
+//        2.62 931 / 985, 3.41 1268 / 1190, 3.81 1291 / 1332; 256 -> 256 the
+//        same way; 128 -> 512 within 1 % above the half.
+//   192  as soon as three 64-column wide tiles a row tile need a third round
+//        (t above 2/3 CUs): 192 -> 192 at 0.6 79 / 89, 0.95 121 / 100, 1.1
+//        194 / 143, 1.7 193 / 187, 2.1 290 / 234, 2.5 292 / 294, 3.5 388 / 366,
+//        6.2 678 / 613; longer rows (384: 1.7 364 / 360, 2.5 549 / 591) by the
+//        last round beyond the first.
+//   96   three a CU, rounds of 1.5 CUs' wide tiles: 96 -> 96 at 0.3 17 / 20, 0.6
+//        31 / 27, 0.95 47 / 31, 1.4 57 / 43, 1.7 61 / 57, 2.1 88 / 68, 2.5 91 /
+//        100 (a round two thirds full, which the CUs that end first take three
+//        at a time), 3.5 121 / 120, 6.2 208 / 188; rows of more than three
+//        chunks (192 -> 96 at 2.1 155 / 126, 3.5 211 / 244, 6.2 369 / 379) only
+//        below two rounds.
+inline bool first_half_round(int64_t t, int64_t per_round) {
+    const int64_t last = t % per_round;
+    return last > 0 && 2 * last <= per_round;
+}
+inline bool small_192(int64_t t, int64_t kch, int64_t cu) {
+    return 3 * t > 2 * cu && (kch <= 6 || t <= cu || first_half_round(t, cu));
+}
+inline bool small_96(int64_t t, int64_t kch, int64_t cu) {
+    const int64_t n = 2 * t, round = 3 * cu;  // 128-row tiles, three a CU
+    if (n <= cu) return false;
+    if (n <= round) return true;
+    if (kch <= 3) return n >= 4 * round || first_half_round(n, round);
+    return n < 2 * round && first_half_round(n, round);
+}
+
 template <typename T, bool Q8, bool PACKED, int NTAPS>
 bool use_small_tiles(const ConvArgs& a) {
     if constexpr (!PACKED || NTAPS == 1) {
@@ -1924,9 +1965,15 @@ bool use_small_tiles(const ConvArgs& a) {
         // short rows into narrow outputs only: with 128 output columns the
         // wide tiles' double-buffered stage wins (C_in 64 -> C_out 128 over
         // 62,710 rows: 53.7 us small, 29.8 us wide; C_in 32: 29.4 / 19.6 us)
-        if (kch <= 2) return a.cout <= 64;
         const int64_t tiles_m = ceil_div(a.n_out, GeoWide::TM);
-        return a.cout % 128 == 0 && tiles_m * (a.cout / 128) > a.num_cu;
+        if constexpr (!Q8 && sizeof(T) == 2) {
+            if (a.cout % 192 == 0 && a.cout % 128 != 0) return small_192(tiles_m * (a.cout / 192), kch, a.num_cu);
+            if (a.cout % 96 == 0 && a.cout % 64 != 0) return small_96(tiles_m * (a.cout / 96), kch, a.num_cu);
+        }
+        if (kch <= 2) return a.cout <= 64;
+        const int64_t t = tiles_m * (a.cout / 128);
+        if (a.cout % 128 != 0 || t <= a.num_cu) return false;
+        return Q8 || sizeof(T) != 2 || first_half_round(t, a.num_cu);
     }
 }
 
@@ -1969,6 +2016,31 @@ bool use_long_tiles(const ConvArgs& a) {
     }
 }
 
+// Class tiles (GeoClass): the 8-tap weight-class conv of a subdivision into 96
+// or 192 channels (an odd multiple of 96), once its 256-row tiles
+// fill half (96) or two thirds (192) of the CUs.  128-row tiles of all the
+// columns, three (two) to a CU, set up in the kernel: the co-resident
+// workgroups hide each other's setup and staging, which a wide tile of 8 taps
+// mostly waits for, and a plan of a table that one conv reads costs more than
+// that (us, wide planned / with its plan / class tiles unplanned): 1,227,072
+// children 192 -> 96 415 / 438 / 384; 138,304 68 / 81 / 58; 35,496 27 / 36 / 25;
+// 153,384 children 768 -> 192 376 / 392 / 297; 61,336 162 / 164 / 121; but
+// 17,288 children 50 / 59 / 79, where 64-column wide tiles fill more CUs.
+template <typename T, bool Q8, bool PACKED, int NTAPS>
+bool use_class_tiles(const ConvArgs& a) {
+    if constexpr (!PACKED || Q8 || NTAPS != 8 || sizeof(T) != 2) {
+        return false;
+    } else {
+        if (a.class_rows <= 0 || a.epi_mode == SPC_EPI_NORM_MOD_SILU || a.cout % 96 != 0 ||
+            a.cout % 128 == 0 || (a.cout % 192 != 0 && a.cout % 64 == 0))
+            return false;
+        if (a.geometry != SPC_TILES_AUTO) return a.geometry == SPC_TILES_SMALL;
+        const int64_t tiles_m = ceil_div(a.n_out, GeoWide::TM);
+        if (a.cout % 192 == 0) return 3 * tiles_m * (a.cout / 192) > 2 * a.num_cu;
+        return 2 * tiles_m * (a.cout / 96) > a.num_cu;
+    }
+}
+
 template <typename T, bool Q8, bool PACKED, int NTAPS>
 hipError_t dispatch_tall(hipStream_t s, const ConvArgs& a) {
     return launch_conv<T, Q8, PACKED, NTAPS, 32, 4, 1, GeoTall>(s, a);
@@ -1989,6 +2061,12 @@ hipError_t dispatch_tn(hipStream_t s, const ConvArgs& a) {
         if constexpr (!Q8 && NTAPS == 27 && sizeof(T) == 2)
             if (use_long_tiles<T, Q8, PACKED, NTAPS>(a))
                 return launch_conv<T, Q8, PACKED, NTAPS, 128, 4, 2, GeoLong>(s, a);
+        if constexpr (!Q8 && NTAPS == 8 && sizeof(T) == 2) {
+            if (use_class_tiles<T, Q8, PACKED, NTAPS>(a)) {
+                if (a.cout % 192 == 0) return launch_conv<T, Q8, PACKED, NTAPS, 192, 2, 2, GeoClass>(s, a);
+                return launch_conv<T, Q8, PACKED, NTAPS, 96, 2, 2, GeoClass>(s, a);
+            }
+        }
         if (use_small_tiles<T, Q8, PACKED, NTAPS>(a)) return dispatch_small<T, Q8, PACKED, NTAPS>(s, a);
     }
     const int64_t tiles_m = ceil_div(a.n_out, GeoWide::TM);

@@ -576,3 +576,67 @@ def test_long_tiles_planned(spc, dev, geo):
         assert msg == ""
         ref = nat.sparse_conv(x, pw, b, idx, ntaps=27, n_out=n, idx_layout=nat.IDX_OFFSET_MAJOR)
         assert torch.equal(y, ref)
+
+
+@pytest.mark.parametrize("dt,cin,cout,n", [
+    ("bf16", 32, 96, 700), ("bf16", 96, 96, 1), ("f16", 192, 96, 257), ("bf16", 192, 192, 640),
+    ("f16", 64, 192, 129)])
+def test_small_96_192_tiles_equal_wide(spc, dev, geo, dt, cin, cout, n):
+    """The small tiles of 96 and 192 columns (128 rows, weights two steps
+    ahead) and, for the 8-tap weight classes, their in-kernel setup, against
+    the wide ones value for value: row remainders, one chunk and several, a
+    tile past the 511-row stage (the per-tap fallback), plain and residual."""
+    import torch
+
+    nat = geo
+    td = torch.bfloat16 if dt == "bf16" else torch.float16
+    print(f"[case] small {cout}-column tiles {dt} N={n} {cin}->{cout}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    r = lambda *s, std=1.0: (torch.randn(s, generator=g, device=dev) * std).to(td)  # noqa: E731
+    n_in = 1500
+    idx = torch.randint(-20, 300, (n, 27), generator=g, device=dev, dtype=torch.int32)
+    idx[: min(n, 128)] += torch.randint(0, 1200, (min(n, 128), 27), generator=g, device=dev,
+                                        dtype=torch.int32)  # the first tile: > 511 rows
+    x, w, b, res = r(n_in, cin), r(cout, 27, cin, std=0.05), r(cout), r(n, cout)
+    pw = nat.pack_weights(w)
+    for e in ({}, {"residual": res}):
+        ys = []
+        for gm in (nat.TILES_WIDE, nat.TILES_SMALL):
+            nat.set_tile_geometry(gm)
+            plan = nat.conv_plan(idx.view(-1), ntaps=27, n_out=n, n_in=n_in)
+            ys += [nat.sparse_conv(x, pw, b, idx.view(-1), ntaps=27, n_out=n, plan=p, **e)
+                   for p in (None, plan)]
+        torch.cuda.synchronize()
+        assert all(torch.equal(ys[0], y) for y in ys)
+    # weight classes: 3 classes of 256 rows, some rows unused
+    w8 = nat.pack_weights(r(24, cout, cin, std=0.1), layout=nat.W_TCK)
+    idx8 = torch.randint(-20, 300, (768, 8), generator=g, device=dev, dtype=torch.int32)
+    idx8[:128] = torch.randint(0, n_in, (128, 8), generator=g, device=dev, dtype=torch.int32)
+    perm = torch.randperm(768, generator=g, device=dev).to(torch.int32)
+    perm[perm >= 700] = -1
+    ys = []
+    for gm in (nat.TILES_WIDE, nat.TILES_SMALL):
+        nat.set_tile_geometry(gm)
+        plan = nat.conv_plan(idx8.view(-1), ntaps=8, n_out=768, n_in=n_in, row_perm=perm)
+        ys += [nat.sparse_conv(x, w8, b, idx8.view(-1), ntaps=8, n_out=768, row_perm=perm, plan=p,
+                               class_rows=256, n_classes=3)[:700] for p in (None, plan)]
+    torch.cuda.synchronize()
+    assert all(torch.equal(ys[0], y) for y in ys)
+
+
+def test_small_tile_rules(spc, dev, geo):
+    """Which rounds of the CUs take the small tiles (256 CUs)."""
+    import torch
+
+    nat = geo
+    k = lambda t, cin, cout, nt=27, cr=0, dt=torch.bfloat16: nat.tile_geometry(  # noqa: E731
+        dt, ntaps=nt, n_out=256 * t, cin=cin, cout=cout, class_rows=cr)
+    S, W = nat.TILES_SMALL, nat.TILES_WIDE
+    assert [k(t, 512, 512) for t in (64, 65, 96, 97, 128, 129)] == [W, S, S, W, W, S]
+    assert [k(t, 192, 192) for t in (170, 171, 300, 640)] == [W, S, S, S]
+    assert [k(t, 384, 192) for t in (171, 384, 385)] == [S, S, W]
+    assert [k(t, 96, 96) for t in (128, 129, 384, 576, 577, 769)] == [W, S, S, S, W, S]
+    assert [k(t, 192, 96) for t in (384, 576, 577, 769)] == [S, S, W, W]
+    assert [k(t, 192, 96, 8, 256 * t) for t in (128, 129)] == [W, S]
+    assert [k(t, 768, 192, 8, 256 * t) for t in (170, 171)] == [W, S]
+    assert k(300, 192, 192, dt=torch.float32) == W
