@@ -528,7 +528,8 @@ int spc_group_norm_silu(spc_stream_t stream, int dtype, const void* x, int64_t n
  * (decoder_mesh.py:82).  scale / shift: f32 [n_batch, cout]
  * holding dtype values (emb_out.type(x.dtype)).  NORM_MOD_SILU needs
  * cout 32, 64 or 128 (one tile covers a whole output row); other widths
- * run the conv and then spc_layernorm_mod_silu. */
+ * run the conv and then spc_layernorm_mod_silu, and so do calls of few rows
+ * in place (the same values up to a rounding that an F32 statistic flips). */
 typedef enum { SPC_EPI_NONE = 0, SPC_EPI_RESIDUAL = 1, SPC_EPI_NORM_MOD_SILU = 2 } spc_epilogue_mode;
 typedef struct {
     int32_t mode;

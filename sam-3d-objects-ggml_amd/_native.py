@@ -132,6 +132,9 @@ class ConvEpilogue(ctypes.Structure):
                 ("residual_rows", ctypes.c_void_p), ("n_residual", ctypes.c_int64)]
 
 
+_NO_EPILOGUE = ConvEpilogue(EPI_NONE, 0.0, None, None, None, None, 0, None, 0)
+
+
 def _check(fn: str, status: int) -> None:
     if status != OK:
         raise SparseConvError(fn, status, lib().spc_last_error().decode(errors="replace"))
@@ -234,6 +237,17 @@ def map_build(coords: torch.Tensor, *, mesh_resolution: int | None = None,
                          _ptr(tm), _ptr(om), _ptr(ms), _ptr(ar), _ptr(mn), _ptr(ws), ws.numel())
     _check("spc_map_build", st)
     return SubmMap(n, tm, om, ms, ar, mn)
+
+
+def map_workspace(n: int, device) -> torch.Tensor:
+    """A workspace for map_build (hash table) over n rows; read_status reads
+    its status word after a build without sync."""
+    return _workspace(lib().spc_map_workspace_bytes(n), device)
+
+
+def read_status(workspace: torch.Tensor) -> None:
+    """Waits for the build and raises its device-side error, if any."""
+    _check("spc_read_status", lib().spc_read_status(_stream(workspace.device), _ptr(workspace)))
 
 
 @dataclass
@@ -599,7 +613,9 @@ def sparse_conv(x: torch.Tensor, weight, bias: torch.Tensor | None,
         bias = bias.contiguous()
     if out is None:
         out = torch.empty((n_out, cout), dtype=x.dtype, device=x.device)
-    epi, keep = _epilogue(x, n_out, cout, residual, norm_mod, residual_rows)  # keep: alive until queued
+    epi, keep = _NO_EPILOGUE, None
+    if residual is not None or norm_mod is not None:
+        epi, keep = _epilogue(x, n_out, cout, residual, norm_mod, residual_rows)  # keep: alive until queued
     if class_rows:
         if not isinstance(weight, PackedWeights):
             raise ValueError("weight classes need PackedWeights")

@@ -466,6 +466,23 @@ std::atomic<int> g_geometry{[] {
 }()};
 int geometry_override() { return g_geometry.load(std::memory_order_relaxed); }
 
+// Whether a SubM conv with the norm epilogue runs as the conv and a row pass
+// over its rounded rows in place (the same steps, spc_layernorm_mod_silu).
+// The epilogue holds whole rows in one column tile: where tiles half as wide
+// still fit a round of the CUs, the conv alone takes them and more CUs.
+// bf16, us (epilogue / conv + pass): 128 -> 128 1,500 rows 50.6 / 22.7, 19,000
+// 51.8 / 33.7, 30,000 52.3 / 39.1, 36,000 53.1 / 52.2, equal above; 512 -> 128
+// 19,000 154 / 94; 64 -> 64 (128-row tiles) 10,000 17.0 / 14.1, 19,000 17.4 /
+// 18.0; 32 -> 32 has no narrower tile.  Packed 16-bit weights, every output row
+// written (no row order), tile geometry by shape.
+bool norm_as_pass(int dtype, int w_dtype, const ConvArgs& a) {
+    if (a.epi_mode != SPC_EPI_NORM_MOD_SILU || !a.packed || a.ntaps != 27 || a.row_perm || a.class_rows > 0 ||
+        a.geometry != SPC_TILES_AUTO || w_dtype != dtype || (dtype != SPC_BF16 && dtype != SPC_F16))
+        return false;
+    if (a.cout == 128) return 2 * ceil_div(a.n_out, GeoWide::TM) <= a.num_cu;
+    return a.cout == 64 && 2 * ceil_div(a.n_out, GeoSmall<27>::TM) <= a.num_cu;
+}
+
 int check_shape(const char* fn, int64_t ntaps, int64_t cin, int64_t cout, bool any_taps = false) {
     const bool taps_ok = any_taps ? (ntaps >= 1 && ntaps <= 4096) : (ntaps == 27 || ntaps == 8 || ntaps == 1);
     if (!taps_ok || cin <= 0 || cout <= 0 || cin % 32 != 0 ||
@@ -806,6 +823,9 @@ int conv_entry(spc_stream_t stream, int dtype, const void* x, int w_dtype, int w
             return SPC_BAD_ARG;
         }
     }
+    // few rows: the conv in narrower column tiles, then the norm as a row pass
+    const bool norm_pass = norm_as_pass(dtype, w_dtype, a);
+    if (norm_pass) a.epi_mode = SPC_EPI_NONE;
     hipError_t e = hipSuccess;
     if (w_dtype == SPC_Q8_0) {
         if (dtype != SPC_BF16) {
@@ -834,6 +854,9 @@ int conv_entry(spc_stream_t stream, int dtype, const void* x, int w_dtype, int w
         return SPC_BAD_ARG;
     }
     if (e != hipSuccess) return hip_status(e, "conv_kernel launch");
+    if (norm_pass)
+        return spc_layernorm_mod_silu(stream, dtype, y, n_out, cout, epi->eps, epi->scale, epi->shift,
+                                      epi->coords, epi->n_batch, y);
     return SPC_OK;
 }
 
@@ -872,6 +895,8 @@ int spc_conv_tile_geometry(int dtype, int w_dtype, int64_t ntaps, int64_t n_out,
     a.epi_mode = epi_mode;
     a.num_cu = device_cu_count();
     a.geometry = geometry_override();
+    a.packed = 1;
+    if (norm_as_pass(dtype, w_dtype, a)) a.epi_mode = SPC_EPI_NONE;
     int g = SPC_TILES_WIDE;
     auto pick = [&](auto t_c, auto q8_c) {
         using T = decltype(t_c);

@@ -561,3 +561,43 @@ def test_subdivide_block_decoder_widths(spc, orc, dev, case):
         assert np.array_equal(y.coords.cpu().numpy(), child)
         assert mr <= MAXREL, (merged, mr)
     blk.merged_taps = True
+
+
+@pytest.mark.parametrize("c,n,plan", [(128, 3000, True), (128, 1, False), (64, 700, False),
+                                      (64, 2000, True)])
+@pytest.mark.parametrize("dt", ["bf16", "f16"])
+def test_norm_pass_equals_epilogue(spc, dev, dt, c, n, plan):
+    """Few rows: the norm epilogue runs as a row pass behind the conv, the same
+    steps on the same rounded rows as the epilogue of a forced geometry; a
+    statistic that differs in its last F32 place may flip a rounding, so
+    nearly every value is equal and none moves by more than a few spacings
+    of the norm's steps (half a spacing each of norm, product, sum and SiLU,
+    relative to their magnitudes)."""
+    import torch
+
+    nat = spc._native
+    td, u = {"bf16": (torch.bfloat16, 2.0 ** -8), "f16": (torch.float16, 2.0 ** -11)}[dt]
+    coords = torch.from_numpy(spc.workloads.random_voxels(n, 18, batches=2, seed=c)).to(dev)
+    n = coords.shape[0]
+    _case(f"norm pass vs epilogue {dt} N={n} C={c}")
+    g = torch.Generator(device="cuda").manual_seed(n)
+    r = lambda *s, std=1.0: (torch.randn(s, generator=g, device=dev) * std).to(td)  # noqa: E731
+    x, w, b = r(n, c), nat.pack_weights(r(c, 27, c, std=0.05)), r(c)
+    m = nat.map_build(coords, outputs="token")
+    p = nat.conv_plan(m.token_major, ntaps=27, n_out=n) if plan else None
+    sc, sh = r(2, c), r(2, c)
+    run = lambda: nat.sparse_conv(x, w, b, m.token_major, ntaps=27, n_out=n, plan=p,  # noqa: E731
+                                  norm_mod=(sc, sh, coords, 1e-6))
+    y = run()
+    conv = nat.sparse_conv(x, w, b, m.token_major, ntaps=27, n_out=n, plan=p)
+    assert torch.equal(y, nat.layernorm_mod_silu(conv, sc, sh, coords, eps=1e-6))
+    nat.set_tile_geometry(nat.TILES_WIDE)
+    try:
+        y0 = run()
+    finally:
+        nat.set_tile_geometry(nat.TILES_AUTO)
+    k = coords[:, 0].long()
+    nrm = torch.nn.functional.layer_norm(conv.double(), (c,), eps=1e-6).abs()
+    mag = nrm * (1 + sc[k].double().abs()) + sh[k].double().abs()
+    assert bool(((y.double() - y0.double()).abs() <= 2 * 4 * u * mag + 2.0 ** -24).all())
+    assert float((y != y0).float().mean()) <= 0.01
