@@ -297,7 +297,7 @@ int spc_sparse_conv_plan(spc_stream_t stream, int dtype, const void* x, int w_dt
 /* Tile geometry of the conv kernel.  Every conv runs on one of four:
  *   SPC_TILES_WIDE   256-row tiles over an 895-row double-buffered stage,
  *                    one 8-wave workgroup per CU (long tiles: wide channels);
- *   SPC_TILES_SMALL  128-row tiles (64 for 8 taps) over a 511-row stage,
+ *   SPC_TILES_SMALL  128-row tiles over a 575-row stage (64 over 511 for 8 taps),
  *                    two or three 4-wave workgroups per CU (short tiles: small
  *                    channel counts, few rows, the stride-2 conv; a stride-2
  *                    conv of up to four 64-byte channel chunks whose tiles

@@ -272,8 +272,10 @@ constexpr int kSegs = 4;        // 16-byte segments per staged 64-byte row chunk
 //             112 KB of A stage, one workgroup of 8 waves per CU -- the wide
 //             convs, where every tile is long.
 //   GeoSmall  128 rows (64 for the 8-tap stride-2 conv, whose 128 coarse
-//             rows reference ~680 fine rows), 511-row stage, swizzled rows,
-//             one buffer: ~42 KB of LDS, three workgroups of 4 waves per CU,
+//             rows reference ~680 fine rows), 575-row stage (511 for 8 taps;
+//             128 children of a shell reference up to 515, and with 511 the one
+//             tile in a thousand past it held its conv back: 126,560 rows 96 ->
+//             96 119 us), swizzled rows, one buffer: ~46 KB of LDS, three workgroups of 4 waves per CU,
 //             which hide each other's staging and setup latency -- the short
 //             tiles of small channel counts, small row counts and stride-2.
 //             (A double-buffered variant measured no faster: stride-2
@@ -359,12 +361,12 @@ struct Geo {
 };
 using GeoWide = Geo<256, 895, 2, true>;
 template <int NTAPS>
-using GeoSmall = Geo<NTAPS == 8 ? 64 : 128, 511, 1, true>;
+using GeoSmall = Geo<NTAPS == 8 ? 64 : 128, NTAPS == 8 ? 511 : 575, 1, true>;
 using GeoTall = Geo<256, 559, 1, true, 895>;
 using GeoQuad = Geo<64, 511, 4, true>;
-using GeoClass = Geo<128, 511, 1, true>;  // GeoSmall<27>'s tile for the 8-tap weight classes
+using GeoClass = Geo<128, 511, 1, true>;  // 128-row tiles of the 8-tap weight classes
 using GeoLong = Geo<320, 1119, 2, true, 1343>;
-static_assert(GeoWide::STAGE == 3584 && GeoSmall<27>::STAGE == 2048 && GeoTall::STAGE == 2240,
+static_assert(GeoWide::STAGE == 3584 && GeoSmall<27>::STAGE == 2304 && GeoTall::STAGE == 2240,
               "stage geometry");
 static_assert(GeoQuad::plan_tile_bytes(8) == GeoSmall<8>::plan_tile_bytes(8) && !GeoQuad::WIDE_PLAN,
               "the four-buffer tiles read the small plan");
@@ -1927,29 +1929,16 @@ hipError_t dispatch_small(hipStream_t s, const ConvArgs& a) {
 //        2.62 931 / 985, 3.41 1268 / 1190, 3.81 1291 / 1332; 256 -> 256 the
 //        same way; 128 -> 512 within 1 % above the half.
 //   192  as soon as three 64-column wide tiles a row tile need a third round
-//        (t above 2/3 CUs): 192 -> 192 at 0.6 79 / 89, 0.95 121 / 100, 1.1
-//        194 / 143, 1.7 193 / 187, 2.1 290 / 234, 2.5 292 / 294, 3.5 388 / 366,
-//        6.2 678 / 613; longer rows (384: 1.7 364 / 360, 2.5 549 / 591) by the
-//        last round beyond the first.
-//   96   three a CU, rounds of 1.5 CUs' wide tiles: 96 -> 96 at 0.3 17 / 20, 0.6
-//        31 / 27, 0.95 47 / 31, 1.4 57 / 43, 1.7 61 / 57, 2.1 88 / 68, 2.5 91 /
-//        100 (a round two thirds full, which the CUs that end first take three
-//        at a time), 3.5 121 / 120, 6.2 208 / 188; rows of more than three
-//        chunks (192 -> 96 at 2.1 155 / 126, 3.5 211 / 244, 6.2 369 / 379) only
-//        below two rounds.
+//        (t above 2/3 CUs): 192 -> 192 at 0.3 40 / 56, 0.6 77 / 88, 0.95 117 /
+//        97, 1.1 192 / 140, 1.7 197 / 182, 2.5 296 / 237, 6.2 719 / 597; 384 ->
+//        192 at 0.6 145 / 169, 0.95 221 / 186, 1.7 370 / 352, 6.2 1417 / 1203.
+//   96   three a CU, above half a round: 96 -> 96 at 0.3 17 / 20, 0.6 31 / 27,
+//        0.95 46 / 31, 1.7 60 / 57, 2.5 92 / 72, 6.2 217 / 172; 32 -> 96 at 6.2
+//        96 / 70; 192 -> 96 at 0.3 28 / 35, 0.6 54 / 50, 1.7 107 / 106, 6.2 362 /
+//        322.
 inline bool first_half_round(int64_t t, int64_t per_round) {
     const int64_t last = t % per_round;
     return last > 0 && 2 * last <= per_round;
-}
-inline bool small_192(int64_t t, int64_t kch, int64_t cu) {
-    return 3 * t > 2 * cu && (kch <= 6 || t <= cu || first_half_round(t, cu));
-}
-inline bool small_96(int64_t t, int64_t kch, int64_t cu) {
-    const int64_t n = 2 * t, round = 3 * cu;  // 128-row tiles, three a CU
-    if (n <= cu) return false;
-    if (n <= round) return true;
-    if (kch <= 3) return n >= 4 * round || first_half_round(n, round);
-    return n < 2 * round && first_half_round(n, round);
 }
 
 template <typename T, bool Q8, bool PACKED, int NTAPS>
@@ -1967,8 +1956,8 @@ bool use_small_tiles(const ConvArgs& a) {
         // 62,710 rows: 53.7 us small, 29.8 us wide; C_in 32: 29.4 / 19.6 us)
         const int64_t tiles_m = ceil_div(a.n_out, GeoWide::TM);
         if constexpr (!Q8 && sizeof(T) == 2) {
-            if (a.cout % 192 == 0 && a.cout % 128 != 0) return small_192(tiles_m * (a.cout / 192), kch, a.num_cu);
-            if (a.cout % 96 == 0 && a.cout % 64 != 0) return small_96(tiles_m * (a.cout / 96), kch, a.num_cu);
+            if (a.cout % 192 == 0 && a.cout % 128 != 0) return 3 * tiles_m * (a.cout / 192) > 2 * a.num_cu;
+            if (a.cout % 96 == 0 && a.cout % 64 != 0) return 2 * tiles_m * (a.cout / 96) > a.num_cu;
         }
         if (kch <= 2) return a.cout <= 64;
         const int64_t t = tiles_m * (a.cout / 128);

@@ -596,7 +596,7 @@ def test_small_96_192_tiles_equal_wide(spc, dev, geo, dt, cin, cout, n):
     n_in = 1500
     idx = torch.randint(-20, 300, (n, 27), generator=g, device=dev, dtype=torch.int32)
     idx[: min(n, 128)] += torch.randint(0, 1200, (min(n, 128), 27), generator=g, device=dev,
-                                        dtype=torch.int32)  # the first tile: > 511 rows
+                                        dtype=torch.int32)  # the first tile: past the stage
     x, w, b, res = r(n_in, cin), r(cout, 27, cin, std=0.05), r(cout), r(n, cout)
     pw = nat.pack_weights(w)
     for e in ({}, {"residual": res}):
@@ -634,9 +634,9 @@ def test_small_tile_rules(spc, dev, geo):
     S, W = nat.TILES_SMALL, nat.TILES_WIDE
     assert [k(t, 512, 512) for t in (64, 65, 96, 97, 128, 129)] == [W, S, S, W, W, S]
     assert [k(t, 192, 192) for t in (170, 171, 300, 640)] == [W, S, S, S]
-    assert [k(t, 384, 192) for t in (171, 384, 385)] == [S, S, W]
-    assert [k(t, 96, 96) for t in (128, 129, 384, 576, 577, 769)] == [W, S, S, S, W, S]
-    assert [k(t, 192, 96) for t in (384, 576, 577, 769)] == [S, S, W, W]
+    assert [k(t, 384, 192) for t in (170, 171, 384)] == [W, S, S]
+    assert [k(t, 96, 96) for t in (128, 129, 384, 640)] == [W, S, S, S]
+    assert [k(t, 192, 96) for t in (128, 129, 1600)] == [W, S, S]
     assert [k(t, 192, 96, 8, 256 * t) for t in (128, 129)] == [W, S]
     assert [k(t, 768, 192, 8, 256 * t) for t in (170, 171)] == [W, S]
     assert k(300, 192, 192, dt=torch.float32) == W
