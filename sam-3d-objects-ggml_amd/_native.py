@@ -239,10 +239,13 @@ def map_build(coords: torch.Tensor, *, mesh_resolution: int | None = None,
     return SubmMap(n, tm, om, ms, ar, mn)
 
 
-def map_workspace(n: int, device) -> torch.Tensor:
-    """A workspace for map_build (hash table) over n rows; read_status reads
-    its status word after a build without sync."""
-    return _workspace(lib().spc_map_workspace_bytes(n), device)
+def map_workspace(n: int, device, dense: tuple | None = None) -> torch.Tensor:
+    """A workspace for map_build over n rows (hash table, or dense =
+    (n_batch, resolution)); read_status reads its status word after a build
+    without sync."""
+    L = lib()
+    return _workspace(L.spc_map_workspace_bytes(n) if dense is None
+                      else L.spc_map_dense_workspace_bytes(n, *dense), device)
 
 
 def read_status(workspace: torch.Tensor) -> None:

@@ -95,7 +95,9 @@ class SparseResBlock3d(nn.Module):
 
     def forward(self, x: SparseTensor, emb: torch.Tensor) -> SparseTensor:
         emb_out = self.emb_layers(emb).type(x.dtype)
-        scale, shift = torch.chunk(emb_out, 2, dim=1)
+        # the halves as F32 in one pass (chunk and two conversions take two)
+        scale, shift = emb_out.reshape(emb_out.shape[0], 2, -1).transpose(0, 1).to(
+            torch.float32, memory_format=torch.contiguous_format).contiguous().unbind(0)
         if self.upsample and self.coarse_rows:
             return self._forward_upsample(x, scale, shift)
         x = self._updown(x)
@@ -104,12 +106,12 @@ class SparseResBlock3d(nn.Module):
         if self.out_channels in (32, 64, 128):
             # one conv tile holds whole output rows: norm2 / modulation / SiLU
             # in the conv's epilogue
-            h = self.conv1.forward_fused(h, norm_mod=(scale.float(), shift.float(),
+            h = self.conv1.forward_fused(h, norm_mod=(scale, shift,
                                                       self.norm2.eps))
         else:
             # wider rows: the conv, then one row pass for norm2 / modulation / SiLU
             h = self.conv1(h)
-            h = h.replace(nat.layernorm_mod_silu(h.feats, scale.float(), shift.float(), h.coords,
+            h = h.replace(nat.layernorm_mod_silu(h.feats, scale, shift, h.coords,
                                                  eps=self.norm2.eps))
         skip = self.skip_connection(x)
         if self.out_channels % 32 == 0:
@@ -140,7 +142,7 @@ class SparseResBlock3d(nn.Module):
         comp = fine.data.cached("subm3_from_coarse", lambda c: nat.compose_rows(m.token_major, rows))
         nm = None
         if self.out_channels in (32, 64, 128):
-            nm = (scale.float(), shift.float(), fine.coords, self.norm2.eps)
+            nm = (scale, shift, fine.coords, self.norm2.eps)
         if self.conv1._use_products(h_c.dtype, n_f, n_c):
             # the fine rows share their coarse rows' products
             y1 = self.conv1._conv_products(h_c, comp, n_f, norm_mod=nm)
@@ -152,7 +154,7 @@ class SparseResBlock3d(nn.Module):
                     epi_mode=nat.EPI_NORM_MOD_SILU if nm else 0)))
             y1 = self.conv1._conv(h_c, comp, n_f, plan, norm_mod=nm)
         if nm is None:
-            y1 = nat.layernorm_mod_silu(y1, scale.float(), shift.float(), fine.coords,
+            y1 = nat.layernorm_mod_silu(y1, scale, shift, fine.coords,
                                         eps=self.norm2.eps)
         h = fine.replace(y1)
         skip = self.skip_connection(x).feats

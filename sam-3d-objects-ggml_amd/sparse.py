@@ -696,7 +696,6 @@ class SparseConv3d(nn.Module, _ConvCore):
         `norm_mod` = (scale, shift, eps) with
         per-batch [B, Cout] scale / shift gives silu(norm(y) * (1 + scale)
         + shift) (structured_latent_flow.py:69-71; Cout 32, 64 or 128)."""
-        spatial_changed = any(s != 1 for s in self.stride) or (self.padding is not None)
         new_shape = torch.Size([x.shape[0], self.conv.out_channels])
         scale = tuple(s * k for s, k in zip(x._scale, self.stride))
         nm = None
@@ -722,8 +721,16 @@ class SparseConv3d(nn.Module, _ConvCore):
                                _plan(x, "down2", d.stride2_taps, 8, d.nc, d.nf))
             spatial = [(s + 1) // 2 for s in x.data.spatial_shape]
             data = SparseTensorData(feats, d.coarse_coords, spatial, x.data.batch_size)
-        out = SparseTensor(data, shape=new_shape, layout=None if spatial_changed else x.layout,
-                           scale=scale, spatial_cache=x._spatial_cache)
+        layout = x.layout
+        if self._kind == "down2":
+            # the coarse rows' batch slices go with the map (computing them
+            # reads the coordinates back to the host: ~100 us of a 145 us
+            # downsample and inverse over 66,779 rows)
+            layout = list(x.data.cached(
+                ("down2_layout", x.shape[0]),
+                lambda c: SparseTensor._batch_slices(d.coarse_coords, x.shape[0])))
+        out = SparseTensor(data, shape=new_shape, layout=layout, scale=scale,
+                           spatial_cache=x._spatial_cache)
         if self._kind == "down2":
             # what SparseInverseConv3d needs to map back to the fine rows
             out.register_spatial_cache(f"conv_{self.stride}_fine_data", x.data)
