@@ -220,7 +220,7 @@ hipError_t launch_norm(hipStream_t s, const void* x, int64_t n, int c, const flo
 // ---- GroupNorm over each batch item's rows (SparseGroupNorm32) ----------
 // Statistics per (item, group) over the item's rows x the group's channels:
 // a partial kernel (one block per (chunk of R rows, item)) writes F64 sums
-// and sums of squares per group; a finalize kernel (one wave per (item,
+// and sums of squares per group; a finalize kernel (one block per (item,
 // group)) adds an item's chunks in a fixed lane-strided order and a fixed
 // shuffle tree.  R depends only on the shape (gn_chunk_rows), so results
 // are deterministic.
@@ -317,19 +317,26 @@ __global__ __launch_bounds__(256) void gn_partial_kernel(const void* __restrict_
     }
 }
 
-// one 64-lane block per (item, group)
-__global__ __launch_bounds__(64) void gn_finalize_kernel(const double* __restrict__ part,
+// One block of eight waves per (item, group): an item's up to 2,048 partials lie
+// 16 bytes in `groups` x 16 apart, so the pass is the latency of its serial
+// loads (one wave, 32 in a row: 13 us at 153,384 rows; the 192 -> 96 block over
+// 15,820 parents 233 -> 221 us, 768 -> 192 over 19,173 737 -> 719, with both passes).
+constexpr int kGnFinalThreads = 512;
+__global__ __launch_bounds__(kGnFinalThreads) void gn_finalize_kernel(const double* __restrict__ part,
                                                          const int64_t* __restrict__ off, int groups,
                                                          int chunks, int rows_per, int cpg, float eps,
                                                          float* __restrict__ stats) {
     const int i = blockIdx.x;
     const int b = i / groups, g = i % groups;
-    const int lane = threadIdx.x;
+    constexpr int NW = kGnFinalThreads / 64;
+    __shared__ double ws[2 * NW];
+    const int lane = threadIdx.x & 63;
     const int64_t rows = off[b + 1] - off[b];
     // never past the partials written (callers pass max_rows >= every item's rows)
     const int used = (int)min<int64_t>((rows + rows_per - 1) / rows_per, chunks);
     double a = 0.0, aa = 0.0;
-    for (int k = lane; k < used; k += 64) {
+#pragma unroll 4
+    for (int k = threadIdx.x; k < used; k += kGnFinalThreads) {
         const double* p = part + (((int64_t)b * chunks + k) * groups + g) * 2;
         a += p[0];
         aa += p[1];
@@ -340,6 +347,18 @@ __global__ __launch_bounds__(64) void gn_finalize_kernel(const double* __restric
         aa += __shfl_xor(aa, o);
     }
     if (lane == 0) {
+        ws[threadIdx.x >> 6] = a;
+        ws[NW + (threadIdx.x >> 6)] = aa;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        a = ws[0];
+        aa = ws[NW];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) {
+            a += ws[w];
+            aa += ws[NW + w];
+        }
         const double cnt = (double)rows * cpg;
         const double mean = cnt > 0 ? a / cnt : 0.0;
         const double var = cnt > 0 ? fmax(aa / cnt - mean * mean, 0.0) : 0.0;
@@ -428,7 +447,7 @@ hipError_t launch_gn_stats(hipStream_t s, const void* x, int c, int groups, cons
     else
         gn_partial_kernel<DT, 1><<<dim3(chunks, n_batch), 256, 0, s>>>(x, c, groups, off, rows_per,
                                                                        part, chunks);
-    gn_finalize_kernel<<<n_batch * groups, 64, 0, s>>>(part, off, groups, chunks, rows_per,
+    gn_finalize_kernel<<<n_batch * groups, kGnFinalThreads, 0, s>>>(part, off, groups, chunks, rows_per,
                                                       c / groups, eps, stats);
     return hipGetLastError();
 }
