@@ -52,7 +52,7 @@ class SlatTables:
         """coords: int32 [nf, 4] (b, x, y, z) on the GPU, 0 <= x,y,z <
         resolution.  Raises SparseConvError where SlatTables::build returns
         false (no rows; coordinates the coarse key cannot hold)."""
-        coords = coords.contiguous()
+        coords, resolution = coords.contiguous(), int(resolution)
         nf = coords.shape[0]
         if nf <= 0:
             raise nat.SparseConvError("SlatTables.build", nat.BAD_SHAPE, "no tokens")

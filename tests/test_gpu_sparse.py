@@ -402,6 +402,18 @@ def test_slat_tables(spc, orc, dev):
         assert np.array_equal(getattr(t, k).cpu().numpy().reshape(v.shape), v), k
 
 
+def test_slat_tables_resolution_forms(spc, dev):
+    """A resolution that int() takes is taken, whichever grid is built."""
+    import torch
+
+    coords = torch.from_numpy(spc.workloads.sphere_shell(20, 7.0)).to(dev)
+    _case(f"SlatTables.build resolution forms N={coords.shape[0]}")
+    a = spc.tables.SlatTables.build(coords, 20)
+    for r in (20.0, np.int64(20), torch.tensor(20)):
+        b = spc.tables.SlatTables.build(coords, r)
+        assert torch.equal(a.conv_fine, b.conv_fine) and torch.equal(a.conv_coarse, b.conv_coarse)
+
+
 def test_mesh_tables(spc, orc, dev):
     import torch
 
