@@ -576,7 +576,7 @@ int spc_sparse_conv_classes(spc_stream_t stream, int dtype, const void* x, const
  * (spc_conv_pack_weights, 27 taps, same dtype); idx token-major [n_out, 27]
  * (entries outside [0, n_in) are missing taps); cin a multiple of 64, cout
  * of 32 (NORM_MOD_SILU: 32, 64 or 128).  x, w, y and workspace 16-byte
- * aligned; workspace holds the products
+ * aligned, the bias at any element; workspace holds the products
  * (spc_conv_products_workspace_bytes: n_in * 27 * cout floats). */
 size_t spc_conv_products_workspace_bytes(int64_t n_in, int64_t cout);
 int spc_sparse_conv_products(spc_stream_t stream, int dtype, const void* x, const void* w,

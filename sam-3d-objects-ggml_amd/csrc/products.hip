@@ -224,12 +224,10 @@ __global__ __launch_bounds__(256) void gather_products_kernel(GatherArgs a, int6
         }
     }
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    if (a.bias) {
-        const u32x2 b = *reinterpret_cast<const u32x2*>(static_cast<const uint16_t*>(a.bias) + c0);
-        acc[0] = M::val(b.x & 0xffffu);
-        acc[1] = M::val(b.x >> 16);
-        acc[2] = M::val(b.y & 0xffffu);
-        acc[3] = M::val(b.y >> 16);
+    if (a.bias) {  // element loads: the bias may lie at any element
+        const uint16_t* b = static_cast<const uint16_t*>(a.bias) + c0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = M::val(b[e]);
     }
     const int64_t ldp = (int64_t)a.ntaps * a.cout;
     const float* pc = a.p + c0;
@@ -343,7 +341,7 @@ int spc_sparse_conv_products(spc_stream_t stream, int dtype, const void* x, cons
         return SPC_BAD_SHAPE;
     }
     if (n_out == 0) return SPC_OK;
-    if (!x || !w || !y || !idx || bad16(x) || bad16(w) || bad16(y) || ((uintptr_t)bias & 7u) != 0) {
+    if (!x || !w || !y || !idx || bad16(x) || bad16(w) || bad16(y)) {
         set_last_error("spc_sparse_conv_products: null / misaligned pointer");
         return SPC_BAD_ARG;
     }

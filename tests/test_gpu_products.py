@@ -87,6 +87,24 @@ def test_products_conv(spc, dev, dtype, n_in, n_out, cin, cout):
         assert float((yn != ref).float().mean()) <= 0.01
 
 
+@pytest.mark.parametrize("at", [0, 1, 2, 3])
+def test_products_conv_bias_at_any_element(spc, dev, at):
+    """A bias that starts at any element of a buffer (a view into flat
+    parameters), as the conv takes it: the same bits as an aligned copy."""
+    import torch
+
+    print(f"[case] products conv bias at element {at}", flush=True)
+    nat = spc._native
+    x, w, b, idx = _setup(100, 300, 64, 64, torch.bfloat16, at)
+    flat = torch.zeros(64 + 8, dtype=torch.bfloat16, device=dev)
+    flat[at:at + 64] = b
+    view = flat[at:at + 64]
+    assert view.data_ptr() % 8 == 2 * at
+    pw = nat.pack_weights(w)
+    y = nat.sparse_conv_products(x, pw, view, idx.reshape(-1), n_out=300)
+    assert torch.equal(y, nat.sparse_conv_products(x, pw, b, idx.reshape(-1), n_out=300))
+
+
 def test_products_conv_equals_conv_on_an_upsampled_level(spc, dev):
     """The up block's route: the same block with the implicit GEMM agrees to
     the F32 order (a rounding step of the 16-bit intermediates at most), and
