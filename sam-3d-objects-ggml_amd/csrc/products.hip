@@ -377,12 +377,22 @@ int spc_sparse_conv_products(spc_stream_t stream, int dtype, const void* x, cons
         g.shift = epi->shift;
         g.coords = epi->coords;
         g.n_batch = epi->n_batch;
-        if ((g.epi_mode == SPC_EPI_RESIDUAL && (!g.residual || bad16(g.residual))) ||
+        if (g.epi_mode == SPC_EPI_NORM_MOD_SILU && cout != 32 && cout != 64 && cout != 128) {
+            set_last_error("spc_sparse_conv_products: the norm epilogue needs cout 32, 64 or 128 "
+                           "(got %lld)", (long long)cout);
+            return SPC_BAD_SHAPE;
+        }
+        // (the conv's own checks)
+        if ((g.epi_mode == SPC_EPI_RESIDUAL &&
+             (!g.residual || bad16(g.residual) ||
+              (g.residual_rows && (g.n_residual < 1 || g.n_residual > INT32_MAX)))) ||
             (g.epi_mode == SPC_EPI_NORM_MOD_SILU &&
              (!g.scale || !g.shift || !g.coords || bad16(g.scale) || bad16(g.shift) || g.n_batch < 1 ||
-              (cout != 32 && cout != 64 && cout != 128))) ||
+              !(g.eps >= 0.0f))) ||
             g.epi_mode < SPC_EPI_NONE || g.epi_mode > SPC_EPI_NORM_MOD_SILU) {
-            set_last_error("spc_sparse_conv_products: bad epilogue");
+            set_last_error("spc_sparse_conv_products: a residual needs a 16-byte aligned pointer and "
+                           "with residual_rows 1 <= n_residual <= INT32_MAX, the norm epilogue 16-byte "
+                           "aligned scale and shift, coords, n_batch >= 1 and eps >= 0");
             return SPC_BAD_ARG;
         }
     }

@@ -8,7 +8,8 @@ out-of-range entries, and each epilogue.
 Bound per element: the F32 sums (27 cin products, any order) are within
 gamma = 27 cin 2^-24 of the F64 one relative to the sum of magnitudes, and
 the result is rounded once to the feature dtype (u = 2^-8 / 2^-11)."""
-import numpy as np
+import ctypes
+
 import pytest
 
 pytestmark = pytest.mark.gpu
@@ -103,6 +104,46 @@ def test_products_conv_bias_at_any_element(spc, dev, at):
     pw = nat.pack_weights(w)
     y = nat.sparse_conv_products(x, pw, view, idx.reshape(-1), n_out=300)
     assert torch.equal(y, nat.sparse_conv_products(x, pw, b, idx.reshape(-1), n_out=300))
+
+
+def test_products_conv_refuses_what_the_conv_refuses(spc, dev):
+    """A negative or NaN eps, residual_rows into no rows and a norm over other
+    widths raise, as in sparse_conv."""
+    import torch
+
+    nat = spc._native
+    x, w, b, idx = _setup(50, 80, 64, 64, torch.bfloat16, 1)
+    pw, coords = nat.pack_weights(w), torch.zeros((80, 4), dtype=torch.int32, device=dev)
+    mod = torch.zeros((1, 64), device=dev)
+    calls = [lambda f, **k: f(norm_mod=(mod, mod, coords, -1.0), **k),
+             lambda f, **k: f(norm_mod=(mod, mod, coords, float("nan")), **k)]
+    both = [lambda **e: nat.sparse_conv_products(x, pw, b, idx.reshape(-1), n_out=80, **e),
+            lambda **e: nat.sparse_conv(x, pw, b, idx.reshape(-1), ntaps=27, n_out=80, **e)]
+    for f in both:
+        for call in calls:
+            print("[case] products conv eps", flush=True)
+            with pytest.raises(nat.SparseConvError):
+                call(f)
+    # the C entries: residual_rows with n_residual 0, and cout 96 with the norm
+    L, s = nat.lib(), torch.cuda.current_stream().cuda_stream
+    y = torch.empty((80, 64), dtype=torch.bfloat16, device=dev)
+    rows = torch.zeros(80, dtype=torch.int32, device=dev)
+    ws = torch.empty(L.spc_conv_products_workspace_bytes(50, 64), dtype=torch.uint8, device=dev)
+    epi = nat.ConvEpilogue(nat.EPI_RESIDUAL, 0.0, y.data_ptr(), None, None, None, 0,
+                           rows.data_ptr(), 0)
+    st = L.spc_sparse_conv_products(s, nat.BF16, x.data_ptr(), pw.data.data_ptr(), None,
+                                    y.data_ptr(), idx.data_ptr(), 80, 50, 64, 64,
+                                    ctypes.byref(epi), ws.data_ptr(), ws.numel())
+    assert st == nat.BAD_ARG
+    p96 = nat.pack_weights(torch.zeros((96, 27, 64), dtype=torch.bfloat16, device=dev))
+    m96 = torch.zeros((1, 96), device=dev)
+    codes = []
+    for f in (lambda **e: nat.sparse_conv_products(x, p96, None, idx.reshape(-1), n_out=80, **e),
+              lambda **e: nat.sparse_conv(x, p96, None, idx.reshape(-1), ntaps=27, n_out=80, **e)):
+        with pytest.raises(nat.SparseConvError) as err:
+            f(norm_mod=(m96, m96, coords, 1e-6))
+        codes.append(err.value.status)
+    assert codes[0] == codes[1]
 
 
 def test_products_conv_equals_conv_on_an_upsampled_level(spc, dev):
