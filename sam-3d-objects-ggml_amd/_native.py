@@ -636,12 +636,19 @@ def sparse_conv(x: torch.Tensor, weight, bias: torch.Tensor | None,
     return out
 
 
+def products_workspace(n_in: int, cout: int, device) -> torch.Tensor:
+    """The products buffer of sparse_conv_products over n_in source rows."""
+    return _workspace(lib().spc_conv_products_workspace_bytes(n_in, cout), device)
+
+
 def sparse_conv_products(x: torch.Tensor, weight: PackedWeights, bias: torch.Tensor | None,
                          idx: torch.Tensor, *, n_out: int, norm_mod: tuple | None = None,
                          residual: torch.Tensor | None = None,
-                         residual_rows: torch.Tensor | None = None) -> torch.Tensor:
+                         residual_rows: torch.Tensor | None = None,
+                         workspace: torch.Tensor | None = None) -> torch.Tensor:
     """The 27-tap conv over a token-major table through per-source-row
-    products (spc_sparse_conv_products); epilogues as in sparse_conv."""
+    products (spc_sparse_conv_products); epilogues as in sparse_conv.
+    `workspace` as products_workspace gives it."""
     _need_gpu(x, bias, idx, weight.data, residual, residual_rows)
     x = x.contiguous()
     dt, (n_in, cin), cout = dtype_code(x.dtype), x.shape, weight.cout
@@ -654,12 +661,10 @@ def sparse_conv_products(x: torch.Tensor, weight: PackedWeights, bias: torch.Ten
         raise ValueError("idx must be int32 [n_out * 27]")
     out = torch.empty((n_out, cout), dtype=x.dtype, device=x.device)
     epi, keep = _epilogue(x, n_out, cout, residual, norm_mod, residual_rows)  # keep: alive until queued
-    L = lib()
-    nbytes = L.spc_conv_products_workspace_bytes(n_in, cout)
-    ws = _workspace(nbytes, x.device)
-    st = L.spc_sparse_conv_products(_stream(x.device), dt, _ptr(x), _ptr(weight.data), _ptr(bias),
-                                    _ptr(out), _ptr(idx), n_out, n_in, cin, cout,
-                                    ctypes.byref(epi), _ptr(ws), nbytes)
+    ws = workspace if workspace is not None else products_workspace(n_in, cout, x.device)
+    st = lib().spc_sparse_conv_products(_stream(x.device), dt, _ptr(x), _ptr(weight.data),
+                                        _ptr(bias), _ptr(out), _ptr(idx), n_out, n_in, cin, cout,
+                                        ctypes.byref(epi), _ptr(ws), ws.numel())
     _check("spc_sparse_conv_products", st)
     return out
 

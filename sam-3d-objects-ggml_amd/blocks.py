@@ -143,10 +143,11 @@ class SparseResBlock3d(nn.Module):
         nm = None
         if self.out_channels in (32, 64, 128):
             nm = (scale, shift, fine.coords, self.norm2.eps)
+        y1 = None
         if self.conv1._use_products(h_c.dtype, n_f, n_c):
             # the fine rows share their coarse rows' products
             y1 = self.conv1._conv_products(h_c, comp, n_f, norm_mod=nm)
-        else:
+        if y1 is None:
             plan = fine.data.cached(("plan", "subm3_from_coarse"), lambda c: nat.conv_plan(
                 comp, ntaps=27, n_out=n_f, n_in=n_c, device=c.device, sections=nat.plan_section(
                     h_c.dtype, ntaps=27, n_out=n_f, cin=_pad32(c1.in_channels),

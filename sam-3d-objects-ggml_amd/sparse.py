@@ -638,17 +638,23 @@ class _ConvCore:
                 and n_out >= 3 * n_in and 108 * n_in * c.out_channels <= 1 << 30)
 
     def _conv_products(self, feats: torch.Tensor, idx: torch.Tensor, n_out: int,
-                       norm_mod: Optional[tuple] = None) -> torch.Tensor:
+                       norm_mod: Optional[tuple] = None) -> Optional[torch.Tensor]:
+        """The conv through its products, or None where their buffer (up to
+        1 GiB) cannot be had: the caller then runs _conv."""
         c = self.conv
         if feats.dim() != 2 or feats.shape[1] != c.in_channels:
             raise ValueError(f"expected feats [N, {c.in_channels}], got {tuple(feats.shape)}")
         nat._need_gpu(feats)
+        try:
+            ws = nat.products_workspace(feats.shape[0], c.out_channels, feats.device)
+        except torch.OutOfMemoryError:
+            return None
 
         def run():
             x = feats.detach().contiguous()
             return nat.sparse_conv_products(x, self._weight_operand(x.dtype, x.device),
                                             self._bias_operand(x.dtype, x.device), idx,
-                                            n_out=n_out, norm_mod=norm_mod)
+                                            n_out=n_out, norm_mod=norm_mod, workspace=ws)
 
         return _run(run, feats, c.weight, c.bias)
 

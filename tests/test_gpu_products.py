@@ -174,3 +174,36 @@ def test_products_conv_equals_conv_on_an_upsampled_level(spc, dev):
     assert not k._use_products(torch.float32, n_f, n_c)
     assert not k._use_products(torch.bfloat16, 2 * n_c, n_c)
     assert not sp.SparseConv3d(128, 128, 3)._use_products(torch.bfloat16, n_f, n_c)
+
+
+def test_up_block_runs_without_room_for_the_products(spc, dev, monkeypatch):
+    """Where the products' buffer cannot be allocated the up block runs the
+    implicit GEMM, with its bits."""
+    import torch
+
+    sp, nat = spc.sparse, spc._native
+    c = torch.from_numpy(spc.workloads.sphere_shell(32, 12.0)).to(dev)
+    ct = sp.SparseDownsample(2)(sp.SparseTensor(torch.zeros((c.shape[0], 32), dtype=torch.bfloat16,
+                                                            device=dev), c))
+    n_c = ct.coords.shape[0]
+    print(f"[case] up block without the products' buffer {n_c} -> {c.shape[0]} rows", flush=True)
+    torch.manual_seed(6)
+    blk = spc.blocks.SparseResBlock3d(512, 64, 128, upsample=True).to(dev).bfloat16()
+    blk.norm1.float()
+    x = ct.replace(torch.randn((n_c, 512), device=dev).bfloat16())
+    emb = torch.randn((1, 64), device=dev).bfloat16()
+    room, need = nat._workspace, 27 * 4 * n_c * 128
+
+    def full(nbytes, device):
+        if nbytes >= need:
+            raise torch.OutOfMemoryError("no room")
+        return room(nbytes, device)
+
+    with torch.no_grad():
+        blk.conv2.conv.weight.normal_(0, 0.02)
+        assert blk.conv1._use_products(torch.bfloat16, c.shape[0], n_c)
+        monkeypatch.setattr(nat, "_workspace", full)
+        y = blk(x, emb).feats
+        monkeypatch.setattr(nat, "_workspace", room)
+        blk.conv1._use_products = lambda *a: False
+        assert torch.equal(y, blk(x, emb).feats)
