@@ -1,0 +1,53 @@
+"""A conv of as many tiles as compute units is one round of them, also when
+its last row tile is partial: such a count takes no more time than one with
+whole tiles (a second round for the one tile would add half or more), up to
+the share that timings of one kernel differ by."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _us(f, reps):
+    import torch
+
+    best = float("inf")
+    for _ in range(5):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        f()
+        a.record()
+        for _ in range(reps):
+            f()
+        b.record()
+        torch.cuda.synchronize()
+        best = min(best, a.elapsed_time(b) / reps * 1e3)
+    return best
+
+
+@pytest.mark.parametrize("n,whole,cin,cout,norm", [
+    (81500, 81920, 256, 128, False),    # 255 full 320-row tiles and a partial one
+    (32500, 32768, 512, 128, True),     # the conv of the norm row pass, 256 64-column tiles
+    (129761, 131072, 256, 128, False),  # two rounds of 256-row tiles
+    (32500, 32768, 256, 256, False)])   # two column tiles a row tile
+def test_partial_tile_takes_no_round_of_its_own(spc, dev, n, whole, cin, cout, norm):
+    import numpy as np
+    import torch
+
+    nat = spc._native
+    c = np.concatenate([spc.workloads.ellipsoid_batch(4, seed=s) + [4 * s, 0, 0, 0]
+                        for s in range(3)]).astype(np.int32)
+    print(f"[case] partial last tile {n} / {whole} rows {cin}->{cout} norm={norm}", flush=True)
+    assert c.shape[0] >= whole
+    g = torch.Generator(device="cuda").manual_seed(1)
+    w = (torch.randn((cout, 27, cin), generator=g, device=dev) * (27 * cin) ** -0.5).bfloat16()
+    b = torch.randn(cout, generator=g, device=dev).bfloat16()
+    pw, mod, us = nat.pack_weights(w), torch.zeros((12, cout), device=dev), []
+    for rows in (n, whole):
+        coords = torch.from_numpy(np.ascontiguousarray(c[:rows])).to(dev)
+        m = nat.map_build(coords, outputs="token")
+        p = nat.conv_plan(m.token_major, ntaps=27, n_out=rows)
+        x = torch.randn((rows, cin), generator=g, device=dev).bfloat16()
+        us.append(_us(lambda: nat.sparse_conv(
+            x, pw, b, m.token_major, ntaps=27, n_out=rows, plan=p,
+            norm_mod=(mod, mod, coords, 1e-6) if norm else None), 30))
+    print(f"[time] {us[0]:.1f} / {us[1]:.1f} us", flush=True)
+    assert us[0] <= 1.2 * us[1], us
