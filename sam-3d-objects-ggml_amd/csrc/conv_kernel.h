@@ -259,10 +259,6 @@ constexpr int kWinWords = 1024;  // dedupe bitmap: 32768 source rows
 constexpr int kWinWordsWide = 2048;
 constexpr int kHashBits = 11;    // wider spans: LDS hash of the tile's source rows
 constexpr int kHashSlots = 1 << kHashBits;  // 64-bit slots: row | rank << 32
-constexpr int kSortCap = 1472;   // distinct rows collected after hashing (> any stage's UCAP)
-constexpr int kSetupScratchWords = 2 * kWinWordsWide > 2 * kHashSlots + 2 * kSortCap
-                                       ? 2 * kWinWordsWide
-                                       : 2 * kHashSlots + 2 * kSortCap;
 constexpr int kSegs = 4;        // 16-byte segments per staged 64-byte row chunk
 
 // Tile geometry: TM output rows per tile, a deduplicated source-row stage of
@@ -327,6 +323,16 @@ struct Geo {
     // union rows a tile may have: the long tiles' may exceed a buffer and
     // take both
     static constexpr int UCAP = LONG ? PUMAX_ : UMAX_;
+    // distinct rows the setup's hash collects (more than UCAP) before it gives
+    // the tile up: the table's probes lengthen as it fills, so no geometry
+    // collects more than it needs (1472 for all: the small tiles' plan of 66,779
+    // shuffled rows 23 us, 15 with 1024; 400,000: 58, 36)
+    static constexpr int SORTCAP = LONG ? 1472 : 1024;
+    // words of setup scratch: the wide bitmap and its word ranks, or the hash
+    // table and its row list
+    static constexpr int SCRATCH = 2 * kWinWordsWide > 2 * kHashSlots + 2 * SORTCAP
+                                       ? 2 * kWinWordsWide
+                                       : 2 * kHashSlots + 2 * SORTCAP;
     static constexpr int PITCH = SW ? 4 : 5;            // 16-byte units per staged row
     static constexpr int UROWCAP = (UCAP + 3) / 4 * 4;  // union-row table (16-byte multiple)
     static constexpr int PUROWCAP = (PUMAX_ + 3) / 4 * 4;  // the plan's union-row table
@@ -398,7 +404,7 @@ constexpr int32_t kPlanMagic = 0x314e4c50;  // header word 3 of every built plan
 
 // Shared-memory arrays of one tile's setup.
 struct TileLds {
-    uint32_t* scratch;  // kSetupScratchWords words: dedupe bitmap + word ranks, or the hash
+    uint32_t* scratch;  // the geometry's SCRATCH words: dedupe bitmap + word ranks, or the hash
     uint16_t* sidx;     // (NTAPS + 1) x TM slot keys; row NTAPS = the zero slot
     uint32_t* tlw;      // kTapWords
     int32_t* urow;      // UMAX source rows of the union slots
@@ -422,6 +428,7 @@ template <int NTAPS, int NT, int PD, typename GEO>
 __device__ __forceinline__ void tile_setup(const ConvArgs& a, int64_t r0, const TileLds& L) {
     constexpr int TM = GEO::TM;
     constexpr int kUMax = GEO::UCAP;
+    constexpr int kSortCap = GEO::SORTCAP;
     constexpr int NW = NT / 64;
     constexpr int NQ = NTAPS * TM;
     constexpr int EPT = (NQ + NT - 1) / NT;
@@ -664,7 +671,7 @@ __device__ __forceinline__ void tile_setup(const ConvArgs& a, int64_t r0, const 
         // the entry order, a wave's 64 lanes wrote TM x 2 bytes apart per tap,
         // into a few LDS banks (the plan of the 1,393,024-row 256^3 level:
         // 10.8 of a tile's 19 us).
-        static_assert(NQ * 2 <= kSetupScratchWords * 4, "slot-key staging fits the scratch");
+        static_assert(NQ * 2 <= GEO::SCRATCH * 4, "slot-key staging fits the scratch");
         lds_barrier();  // every thread is done with the bitmap / hash
         uint16_t* stg = reinterpret_cast<uint16_t*>(L.scratch);
 #pragma unroll
@@ -705,7 +712,7 @@ __device__ __forceinline__ void tile_setup(const ConvArgs& a, int64_t r0, const 
 template <int NTAPS, typename GEO>
 __global__ __launch_bounds__(512) void conv_plan_kernel(ConvArgs a, char* plan) {
     constexpr int TM = GEO::TM;
-    __shared__ __attribute__((aligned(16))) uint32_t scratch[kSetupScratchWords];
+    __shared__ __attribute__((aligned(16))) uint32_t scratch[GEO::SCRATCH];
     __shared__ __attribute__((aligned(16))) uint16_t sidx[(NTAPS + 1) * TM];
     __shared__ __attribute__((aligned(16))) uint32_t tlw[kTapWords];
     __shared__ __attribute__((aligned(16))) int32_t urow[GEO::UROWCAP];
@@ -780,7 +787,7 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
                   "wave geometry");
     static_assert(!Q8 || ES == 2, "Q8_0 weights feed 16-bit MFMA operands");
     static_assert(NTAPS <= 32, "tap mask is 32-bit");
-    static_assert(kSetupScratchWords * 4 <= ABYTES, "setup scratch aliases the A stage");
+    static_assert(GEO::SCRATCH * 4 <= ABYTES, "setup scratch aliases the A stage");
     static_assert(PD == 4, "the step groups pack four taps per word");
     static_assert(NBUF == 1 || NBUF == 2 || NBUF == 4, "one, two or four A buffers");
 
@@ -794,7 +801,7 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
     int32_t* const urow = GEO::LONG ? reinterpret_cast<int32_t*>(Au + NBUF * STAGE) - GEO::UROWCAP : urow_own;
     static_assert(!GEO::LONG || ((GEO::UCAP + 1) * 4 + 63) / 64 * 64 + GEO::UROWCAP / 4 <= NBUF * STAGE,
                   "the union rows lie past a tile taking both buffers");
-    static_assert(!GEO::LONG || kSetupScratchWords * 4 + GEO::UROWCAP * 4 <= ABYTES,
+    static_assert(!GEO::LONG || GEO::SCRATCH * 4 + GEO::UROWCAP * 4 <= ABYTES,
                   "the union rows lie past the setup scratch");
     __shared__ __attribute__((aligned(16))) int32_t srow[TM];        // output row of each tile row
     __shared__ int32_t wsum[NW];
