@@ -476,6 +476,8 @@ def convert(x: torch.Tensor, dtype: torch.dtype, out: torch.Tensor | None = None
 
 TILES_AUTO, TILES_WIDE, TILES_SMALL, TILES_TALL, TILES_LONG = 0, 1, 2, 3, 4
 PLAN_WIDE, PLAN_SMALL, PLAN_LONG = 1, 2, 4
+# the row counts whose 27-tap plans have a PLAN_LONG section
+LONG_ROWS = range(256 * 256 + 1, 256 * 320 + 1)
 
 
 def tile_geometry(dtype: torch.dtype, *, ntaps: int, n_out: int, cin: int, cout: int,

@@ -27,8 +27,8 @@ import torch.nn as nn
 
 from . import _native as nat
 from .sparse import (SparseConv3d, SparseDownsample, SparseGroupNorm32, SparseLinear, SparseSiLU,
-                     SparseSubdivide, SparseTensor, SparseUpsample, _pad32, _run, _subm_map,
-                     batch_offsets, max_item_rows)
+                     SparseSubdivide, SparseTensor, SparseUpsample, _LONG_PLAN, _pad32, _run,
+                     _subm_map, batch_offsets, max_item_rows)
 
 __all__ = ["LayerNorm32", "SparseResBlock3d", "SparseSubdivideBlock3d"]
 
@@ -287,7 +287,9 @@ class SparseSubdivideBlock3d(nn.Module):
         h.data.cached("subm3", lambda c: cm)  # conv2's map: the same child coordinates
         plan2 = plan(cm.token_major, _pad32(c2.out_channels), ntaps=27, n_out=nc,
                      cin=_pad32(c2.in_channels), epi_mode=nat.EPI_RESIDUAL)
-        h.data.cached(("plan", "subm3"), lambda c: plan2)
+        key2 = _LONG_PLAN if nc in nat.LONG_ROWS and conv2._reads_long(dt, nc, nat.EPI_NONE) \
+            else ("plan", "subm3")
+        h.data.cached(key2, lambda c: plan2)
         h = h.replace(nat.group_norm_silu(h.feats, 8 * offs, gn1.num_groups, gn1.weight, gn1.bias,
                                           gn1.eps, silu=True, max_rows=8 * rows_max))
         # the skip on the parent rows (a 1x1x1 conv is row-wise), added to
@@ -299,5 +301,5 @@ class SparseSubdivideBlock3d(nn.Module):
         else:
             y = conv2(h) + h.replace(nat.gather_rows(skip, parent))
         if plan2 is None:  # later convs over these rows build their own
-            y.data.indice_dict.pop(("plan", "subm3"), None)
+            y.data.indice_dict.pop(key2, None)
         return y

@@ -6,6 +6,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 
 #include "conv_kernel.h"
 
@@ -17,9 +18,10 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 // Clears the marker of `tiles` plan tiles (a section its builder skipped):
 // convs over them set their tiles up themselves.
-__global__ void plan_unmark_kernel(char* plan, int64_t tiles, int64_t tile_bytes) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < tiles) reinterpret_cast<int32_t*>(plan + t * tile_bytes)[3] = 0;
+__global__ void plan_unmark_kernel(PlanMarks m, PlanMarks also) {
+    const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    m.clear(t);
+    also.clear(t);
 }
 
 template <typename T, bool Q8>
@@ -663,27 +665,37 @@ int spc_conv_plan_sections(spc_stream_t stream, const int32_t* idx, int idx_layo
     a.idx_layout = idx_layout;
     a.ntaps = (int32_t)ntaps;
     // the wide tiles' plans, then the small tiles', then the long tiles' where
-    // the row count has them; a section not asked for
-    // has its tiles' markers cleared (its convs set their tiles up themselves)
+    // the row count has them; a section not asked for has its tiles' markers
+    // cleared (its convs set their tiles up themselves)
     char* pl = static_cast<char*>(plan);
     char* ps = pl + plan_wide_bytes(n_out, (int)ntaps);
-    auto section = [&](auto ntaps_c, auto geo_c, char* base, bool build) {
+    auto section = [&](auto ntaps_c, auto geo_c, char* base, bool build, PlanMarks also = {}) {
         constexpr int NT_ = decltype(ntaps_c)::value;
         using G = decltype(geo_c);
         const int64_t tiles = ceil_div(n_out, G::TM);
+        if constexpr (NT_ == 27 && std::is_same_v<G, GeoWide>) {
+            if (build && also.base) {
+                conv_plan_kernel<NT_, G, true><<<(unsigned)tiles, 512, 0, s>>>(a, base, also);
+                return;
+            }
+        }
         if (build)
-            conv_plan_kernel<NT_, G><<<(unsigned)tiles, 512, 0, s>>>(a, base);
+            conv_plan_kernel<NT_, G><<<(unsigned)tiles, 512, 0, s>>>(a, base, also);
         else
             plan_unmark_kernel<<<(unsigned)ceil_div(tiles, 256), 256, 0, s>>>(
-                base, tiles, G::plan_tile_bytes(NT_));
+                PlanMarks{base, tiles, G::plan_tile_bytes(NT_)}, also);
     };
     const bool w = sections & SPC_PLAN_WIDE, sm = sections & SPC_PLAN_SMALL;
     if (ntaps == 27) {
-        section(std::integral_constant<int, 27>{}, GeoWide{}, pl, w);
+        // a long section that is not asked for costs no launch of its own
+        char* plong = ps + plan_small_bytes(n_out, 27);
+        const bool has_long = plan_long_bytes(n_out, 27) > 0;
+        const bool lg = has_long && (sections & SPC_PLAN_LONG) != 0;
+        section(std::integral_constant<int, 27>{}, GeoWide{}, pl, w,
+                has_long && !lg ? PlanMarks{plong, ceil_div(n_out, GeoLong::TM), GeoLong::plan_tile_bytes(27)}
+                                : PlanMarks{});
         section(std::integral_constant<int, 27>{}, GeoSmall<27>{}, ps, sm);
-        if (plan_long_bytes(n_out, 27) > 0)
-            section(std::integral_constant<int, 27>{}, GeoLong{}, ps + plan_small_bytes(n_out, 27),
-                    (sections & SPC_PLAN_LONG) != 0);
+        if (lg) section(std::integral_constant<int, 27>{}, GeoLong{}, plong, true);
     } else if (ntaps == 8) {
         section(std::integral_constant<int, 8>{}, GeoWide{}, pl, w);
         section(std::integral_constant<int, 8>{}, GeoSmall<8>{}, ps, sm);

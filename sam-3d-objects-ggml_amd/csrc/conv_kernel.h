@@ -707,10 +707,21 @@ __device__ __forceinline__ void tile_setup(const ConvArgs& a, int64_t r0, const 
     lds_barrier();
 }
 
+// The markers of a plan section's tiles.
+struct PlanMarks {
+    char* base;
+    int64_t tiles;
+    int64_t tile_bytes;
+    __device__ void clear(int64_t t) const {
+        if (t < tiles) reinterpret_cast<int32_t*>(base + t * tile_bytes)[3] = 0;
+    }
+};
+
 // One block per row tile of geometry GEO: runs the tile setup once and
-// stores it, so every conv over the same index table skips it.
-template <int NTAPS, typename GEO>
-__global__ __launch_bounds__(512) void conv_plan_kernel(ConvArgs a, char* plan) {
+// stores it, so every conv over the same index table skips it.  UNMARK: block
+// t also clears marker t of a section of no more tiles that is not built.
+template <int NTAPS, typename GEO, bool UNMARK = false>
+__global__ __launch_bounds__(512) void conv_plan_kernel(ConvArgs a, char* plan, PlanMarks unmark) {
     constexpr int TM = GEO::TM;
     __shared__ __attribute__((aligned(16))) uint32_t scratch[GEO::SCRATCH];
     __shared__ __attribute__((aligned(16))) uint16_t sidx[(NTAPS + 1) * TM];
@@ -721,6 +732,7 @@ __global__ __launch_bounds__(512) void conv_plan_kernel(ConvArgs a, char* plan) 
     __shared__ int32_t misc[8];
     const TileLds L{scratch, sidx, tlw, urow, srow, wsum, misc};
     const int64_t tm = blockIdx.x;
+    if (UNMARK && threadIdx.x == 0) unmark.clear(tm);
     tile_setup<NTAPS, 512, 4, GEO>(a, tm * TM, L);
     char* pt = plan + tm * GEO::plan_tile_bytes(NTAPS);
     int32_t* hdr = reinterpret_cast<int32_t*>(pt);

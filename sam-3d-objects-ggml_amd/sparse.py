@@ -394,10 +394,16 @@ def _resolution(x: SparseTensor) -> int:
     return max(2, max(x.data.spatial_shape) if x.data.spatial_shape else 2)
 
 
+# cache key of a SubM table's plan for the 320-row tiles
+_LONG_PLAN = ("plan", "subm3", "long")
+
+
 def _plan(x: SparseTensor, key, idx, ntaps: int, n_out: int, n_in: int):
-    """Tile plan of an index table, cached with the coordinates like the maps."""
+    """Tile plan of an index table, cached with the coordinates like the maps
+    (without the 320-row tiles' section, which few convs read: _LONG_PLAN)."""
     return x.data.cached(("plan", key), lambda c: nat.conv_plan(
-        idx, ntaps=ntaps, n_out=n_out, n_in=n_in, device=c.device))
+        idx, ntaps=ntaps, n_out=n_out, n_in=n_in, device=c.device,
+        sections=nat.PLAN_WIDE | nat.PLAN_SMALL))
 
 
 def _downsample_map(x: SparseTensor) -> nat.DownsampleMap:
@@ -618,6 +624,15 @@ class _ConvCore:
 
         return _run(run, feats, c.weight, c.bias)
 
+    def _reads_long(self, dtype: torch.dtype, n_out: int, epi_mode: int) -> bool:
+        """Whether a 27-tap conv of n_out rows (in nat.LONG_ROWS) reads its plan's
+        320-row section: 128-column tiles only (Q8_0 weights are expanded to 16
+        bits at such row counts)."""
+        c = self.conv
+        cout = _pad32(c.out_channels)
+        return cout % 128 == 0 and nat.plan_section(
+            dtype, ntaps=27, n_out=n_out, cin=_pad32(c.in_channels), cout=cout,
+            epi_mode=epi_mode) == nat.PLAN_LONG
 
     def _use_products(self, dtype: torch.dtype, n_out: int, n_in: int) -> bool:
         """Whether a 27-tap conv of n_out rows over n_in source rows forms
@@ -713,7 +728,13 @@ class SparseConv3d(nn.Module, _ConvCore):
         if self._kind == "subm3":
             m = _subm_map(x)
             n = x.feats.shape[0]
-            feats = self._conv(x.feats, m.token_major, n, _plan(x, "subm3", m.token_major, 27, n, n),
+            if n in nat.LONG_ROWS and self._reads_long(
+                    x.feats.dtype, n, nat.EPI_NONE if nm is None else nat.EPI_NORM_MOD_SILU):
+                plan = x.data.cached(_LONG_PLAN, lambda c: nat.conv_plan(
+                    m.token_major, ntaps=27, n_out=n, device=c.device, sections=nat.PLAN_LONG))
+            else:
+                plan = _plan(x, "subm3", m.token_major, 27, n, n)
+            feats = self._conv(x.feats, m.token_major, n, plan,
                                residual=residual, norm_mod=nm, residual_rows=residual_rows)
             data = x.data.replace_feature(feats)
         elif self._kind == "subm1":

@@ -88,6 +88,36 @@ def test_subm3_bf16_module_map_cached(spc, orc, dev):
     assert y.feats.shape == (n, 128) and y.layout == xt.layout
 
 
+def test_plan_sections_are_built_by_the_convs_that_read_them(spc, dev, monkeypatch):
+    """The 320-row tiles' plan is built for the first conv that runs them, and
+    by no other; convs of either kind in any order read their own section."""
+    import torch
+
+    nat, sp = spc._native, _sp(spc)
+    c = spc.workloads.ellipsoid_batch(4)
+    extra = c[c[:, 0] == 0] + np.array([4, 0, 0, 0], c.dtype)
+    coords = torch.from_numpy(np.concatenate([c, extra])[:66000]).to(dev)
+    n = coords.shape[0]
+    _case(f"plan sections N={n}")
+    built, real = [], nat.conv_plan
+    monkeypatch.setattr(nat, "conv_plan", lambda *a, **k: (built.append(k["sections"]),
+                                                           real(*a, **k))[1])
+    torch.manual_seed(3)
+    convs = {w: sp.SparseConv3d(64, w, 3).to(dev).bfloat16() for w in (64, 128)}
+    x = torch.randn((n, 64), device=dev).bfloat16()
+    base, own = nat.PLAN_WIDE | nat.PLAN_SMALL, nat.PLAN_LONG
+    for order, want in (((64, 128, 64, 128), [base, own]), ((128, 128), [own])):
+        xt = sp.SparseTensor(x, coords.clone())
+        built.clear()
+        with torch.no_grad():
+            ys = {w: convs[w](xt).feats for w in order}
+        assert built == want
+        m = nat.map_build(coords, outputs="token")
+        for w, y in ys.items():
+            cw, b = convs[w]._weight_operand(x.dtype, x.device), convs[w].conv.bias.detach()
+            assert torch.equal(y, nat.sparse_conv(x, cw, b, m.token_major, ntaps=27, n_out=n))
+
+
 def test_subm1_raw_view(spc, orc, dev):
     """1x1x1: the saved [Cout,1,1,1,Cin] buffer is read as (Cin, Cout)
     (SRC/mesh_decoder_graph.cpp:349-376); Cin != Cout so a transposed
