@@ -636,21 +636,28 @@ class _ConvCore:
 
     def _use_products(self, dtype: torch.dtype, n_out: int, n_in: int) -> bool:
         """Whether a 27-tap conv of n_out rows over n_in source rows forms
-        each (source row, tap) product once (_conv_products).  Measured on
-        shells, 128 output channels, bf16, with the norm epilogue, in us (conv
-        / products), n_out 5.3 n_in: 66,779 rows C_in 2048 1173 / 215, 512
-        324 / 116, 256 183 / 97, 128 113 / 89; 1,512 rows 2048 537 / 51, 256
-        83 / 22.  Without an epilogue C_in 256 gains (131 / 88; 49 / 31 at
-        19,173 rows) and 128 loses (77 / 87; 28.4 / 29.7), so the line is at
-        256.  The dense product multiplies all 27 taps of every source row,
-        the conv ~27 of every output row: below about 3 output rows to a
-        source row the products' F32 traffic is no longer paid for.  Their
-        buffer is held to 1 GiB."""
+        each (source row, tap) product once (_conv_products).  Products
+        multiply all 27 taps of every source row and pay F32 traffic for every
+        output column; the conv multiplies ~27 taps of every output row.
+        Measured on shells and thinned shells, bf16, us (conv / products; the
+        norm epilogue at 32, 64 and 128 columns):
+          12,516 -> 66,779 rows (5.3 a source row), to 128 columns: C_in 256
+          121 / 97, 512 219 / 114, 2048 726 / 211; 284 -> 1,512: 2048 537 / 51;
+          C_in 128 loses without an epilogue (77 / 87), so the line is at 256;
+          11,722 -> 40,167 rows (3.4): C_in 256 to 64 columns 52 / 50, 128 92 /
+          80, 192 103 / 110, 256 129 / 165, 512 214 / 329; C_in 384 to 256
+          190 / 180, 512 312 / 359; C_in 512 to 512 413 / 391 (3.0 a source
+          row: 399 / 375) -- below 512 input channels only narrow outputs gain
+          at every ratio taken.
+        Below about 3 output rows to a source row the F32 traffic is no longer
+        paid for.  The products' buffer is held to 1 GiB."""
         c = self.conv
+        cin, cout = c.in_channels, c.out_channels
         return (dtype in (torch.bfloat16, torch.float16) and self._q8 is None
-                and c.in_channels >= 256 and c.in_channels % 64 == 0 and c.out_channels % 32 == 0
-                and 54 * c.in_channels * c.out_channels < 1 << 31
-                and n_out >= 3 * n_in and 108 * n_in * c.out_channels <= 1 << 30)
+                and cin >= 256 and cin % 64 == 0 and cout % 32 == 0
+                and (cin >= 512 or cout <= cin - 128)
+                and 54 * cin * cout < 1 << 31
+                and n_out >= 3 * n_in and 108 * n_in * cout <= 1 << 30)
 
     def _conv_products(self, feats: torch.Tensor, idx: torch.Tensor, n_out: int,
                        norm_mod: Optional[tuple] = None) -> Optional[torch.Tensor]:

@@ -180,3 +180,23 @@ def test_kernel_ops_refuse_cpu_tensors(sp, spc):
         sp.SparseUpsample(2)(x32)
     with pytest.raises(RuntimeError, match="GPU only"):
         spc.tables.SlatTables.build(x.coords)
+
+
+def test_products_rule(spc):
+    """Which upsampled convs run as products shared between a source row's
+    children: from 256 input channels on, below 512 only into outputs 128
+    channels narrower (wider ones lose to the implicit GEMM at 3 to 5 output
+    rows a source row), 16-bit, three output rows to a source row, 1 GiB."""
+    import torch
+
+    def rule(cin, cout, n_out=40000, n_in=12000, dt=torch.bfloat16):
+        return spc.sparse.SparseConv3d(cin, cout, 3)._use_products(dt, n_out, n_in)
+
+    took = {cin: [c for c in (32, 64, 96, 128, 192, 256, 320, 512) if rule(cin, c)]
+            for cin in (128, 192, 256, 320, 384, 512, 544)}
+    assert took == {128: [], 192: [], 256: [32, 64, 96, 128], 320: [32, 64, 96, 128, 192],
+                    384: [32, 64, 96, 128, 192, 256],
+                    512: [32, 64, 96, 128, 192, 256, 320, 512], 544: []}
+    assert rule(2048, 128) and rule(2048, 128, dt=torch.float16)
+    assert not rule(2048, 128, dt=torch.float32) and not rule(2048, 128, 40000, 13334)
+    assert rule(512, 512, 10 ** 6, 19418) and not rule(512, 512, 10 ** 6, 19419)
