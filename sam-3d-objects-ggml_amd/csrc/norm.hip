@@ -80,13 +80,15 @@ struct NormMod {
 };
 
 // G lanes per row, NV runs of 4 per lane (c <= 4 * G * NV), R rows per lane
-// group (rows r, r + groups, ...: R independent reductions in flight)
+// group (rows r, r + groups, ...: R independent reductions in flight).  y may
+// be x (no __restrict__ on either): a lane has all its rows' elements in
+// registers before it stores one, and no lane reads another's.
 template <int DT, int G, int NV, int R>
-__global__ __launch_bounds__(256) void layernorm_silu_kernel(const void* __restrict__ x, int64_t n,
+__global__ __launch_bounds__(256) void layernorm_silu_kernel(const void* x, int64_t n,
                                                              int c, const float* __restrict__ gamma,
                                                              const float* __restrict__ beta,
-                                                             float eps, int silu,
-                                                             void* __restrict__ y, NormMod mod) {
+                                                             float eps, int silu, void* y,
+                                                             NormMod mod) {
     using E = Elem<DT>;
     const int lane = threadIdx.x & 63;
     constexpr int GPB = 256 / G;  // row groups per block

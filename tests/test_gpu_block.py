@@ -151,6 +151,28 @@ def test_layernorm_mod_silu(spc, orc, dev, dt, c):
         assert np.mean(got == ref) >= 0.98
 
 
+@pytest.mark.parametrize("dt", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("c", [4, 64, 128, 256, 1024, 2048])
+def test_layernorm_in_place(spc, dev, dt, c):
+    """Both row passes over their own input (the few-row norm epilogue's form):
+    the bits of a call into another buffer."""
+    import torch
+
+    _case(f"layernorm in place {dt} c={c}")
+    nat = spc._native
+    td = {"bf16": torch.bfloat16, "f16": torch.float16, "f32": torch.float32}[dt]
+    n = 1003
+    g = torch.Generator(device="cuda").manual_seed(c)
+    x = torch.randn((n, c), generator=g, device=dev).to(td)
+    a, b = (torch.randn((2, c), generator=g, device=dev) for _ in range(2))
+    coords = torch.zeros((n, 4), dtype=torch.int32, device=dev)
+    coords[400:, 0] = 1
+    for f in (lambda t, **k: nat.layernorm_mod_silu(t, a, b, coords, **k),
+              lambda t, **k: nat.layernorm_silu(t, a[0], b[0], **k)):
+        y, t = f(x), x.clone()
+        assert f(t, out=t) is t and torch.equal(t, y)
+
+
 def _block_params(blk):
     p = {"norm1_w": blk.norm1.weight, "norm1_b": blk.norm1.bias,
          "conv1_w": blk.conv1.conv.weight, "conv1_b": blk.conv1.conv.bias,
