@@ -258,14 +258,14 @@ class SparseSubdivideBlock3d(nn.Module):
         c1, c2 = conv1.conv, conv2.conv
         dt = x.feats.dtype
         # the plans are rebuilt per call: only the tile geometry each conv runs,
-        # and none for small tiles of all the columns (96 or 192), which each
-        # read it once and set up in the kernel behind each other's loops
-        # (1,227,072 rows 96 -> 96: plan + conv 661 us, conv alone 626)
-        def plan(idx, cout, **shape):
-            g = nat.tile_geometry(dt, ntaps=shape["ntaps"], n_out=shape["n_out"], cin=shape.pop("cin"),
-                                  cout=cout, class_rows=shape.pop("class_rows", 0),
-                                  epi_mode=shape.pop("epi_mode", 0))
-            if g == nat.TILES_SMALL and cout in (96, 192):
+        # none for the class tiles, which read no plan, and none for small tiles
+        # of all the columns (96 or 192), which each read it once and set up in
+        # the kernel behind each other's loops (1,227,072 rows 96 -> 96: plan +
+        # conv 661 us, conv alone 626)
+        def plan(idx, cout, *, cin, class_rows=0, epi_mode=0, **shape):
+            g = nat.tile_geometry(dt, ntaps=shape["ntaps"], n_out=shape["n_out"], cin=cin, cout=cout,
+                                  class_rows=class_rows, epi_mode=epi_mode)
+            if g == nat.TILES_SMALL and (class_rows or cout in (96, 192)):
                 return None
             return nat.conv_plan(idx, sections=nat.geometry_section(g), **shape)
 

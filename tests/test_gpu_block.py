@@ -623,3 +623,25 @@ def test_norm_pass_equals_epilogue(spc, dev, dt, c, n, plan):
     mag = nrm * (1 + sc[k].double().abs()) + sh[k].double().abs()
     assert bool(((y.double() - y0.double()).abs() <= 2 * 4 * u * mag + 2.0 ** -24).all())
     assert float((y != y0).float().mean()) <= 0.01
+
+
+@pytest.mark.parametrize("cin,cout,n,want", [(96, 288, 2500, [27]), (96, 96, 5000, []),
+                                             (96, 288, 300, [8, 27])])
+def test_subdivide_block_plans(spc, dev, monkeypatch, cin, cout, n, want):
+    """The plans a subdivide block builds: none that its convs do not read (the
+    class tiles of 96, 192 and 288 columns set up in the kernel)."""
+    import torch
+
+    nat, sp = spc._native, spc.sparse
+    c = torch.from_numpy(spc.workloads.sphere_shell()[:n]).to(dev)
+    _case(f"subdivide block plans N={n} {cin}->{cout}")
+    built, real = [], nat.conv_plan
+    blk = spc.blocks.SparseSubdivideBlock3d(cin, 64, cout).to(dev).bfloat16()
+    for m in blk.modules():
+        if isinstance(m, torch.nn.GroupNorm):
+            m.float()
+    monkeypatch.setattr(nat, "conv_plan", lambda *a, **k: (built.append(k["ntaps"]),
+                                                           real(*a, **k))[1])
+    with torch.no_grad():
+        blk(sp.SparseTensor(torch.randn((n, cin), device=dev).bfloat16(), c))
+    assert [t for t in built if t > 1] == want
