@@ -310,11 +310,16 @@ int spc_sparse_conv_plan(spc_stream_t stream, int dtype, const void* x, int w_dt
  *                    tile of up to 1343 rows takes both buffers as one):
  *                    16-bit convs of C_out 128 that 256-row tiles would
  *                    leave a nearly empty second round of the CUs.
- * All give the same results.  By default (SPC_TILES_AUTO) each conv picks
+ * All sum a row's products in the same order and give the same results; the
+ * norm epilogue alone may differ by a rounding (by shape, calls of few rows run
+ * it as a row pass behind the conv, see spc_conv_epilogue; under a forced
+ * geometry it runs in the conv).  By default (SPC_TILES_AUTO) each conv picks
  * by shape; spc_conv_set_tile_geometry forces one for every later conv of
  * the process (measurements, tests; initially from the environment
  * variable SPC_CONV_GEOMETRY = "wide" / "small" / "tall" / "long").  The small tiles
- * apply to packed weights with 27 or 8 taps, the tall ones to packed
+ * apply to packed weights with 27 or 8 taps (of the weight classes by shape
+ * only to 16-bit ones of 8 taps into an odd multiple of 96 columns: 128-row
+ * class tiles over a 511-row stage, which read no plan), the tall ones to packed
  * weights with 27 taps and C_out a multiple of 32, without the norm
  * epilogue or weight classes, the long ones to packed 16-bit weights with
  * 27 taps and C_out a multiple of 128 (elsewhere a forced geometry that does not
@@ -329,8 +334,9 @@ int spc_sparse_conv_plan(spc_stream_t stream, int dtype, const void* x, int w_dt
 int spc_conv_set_tile_geometry(int geometry);
 /* The geometry (SPC_TILES_WIDE / SMALL / TALL / LONG) a conv with packed weights
  * and these arguments runs now (epi_mode a spc_epilogue_mode, class_rows 0
- * without weight classes); SPC_TILES_SMALL reads the small plan section,
- * SPC_TILES_LONG the long one, the others the wide one. */
+ * without weight classes); SPC_TILES_SMALL reads the small plan section (for
+ * weight classes of an odd multiple of 96 columns none: a plan passed to them is
+ * ignored), SPC_TILES_LONG the long one, the others the wide one. */
 int spc_conv_tile_geometry(int dtype, int w_dtype, int64_t ntaps, int64_t n_out, int64_t cin,
                            int64_t cout, int64_t class_rows, int epi_mode);
 

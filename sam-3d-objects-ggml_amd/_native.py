@@ -493,7 +493,8 @@ def plan_section(dtype: torch.dtype, *, ntaps: int, n_out: int, cin: int, cout: 
                  q8: bool = False, class_rows: int = 0, epi_mode: int = 0) -> int:
     """The plan section (PLAN_WIDE / PLAN_SMALL / PLAN_LONG) a packed-weight
     conv with these arguments reads: the small and the long tiles read their
-    own, the wide and the tall tiles the wide one."""
+    own, the wide and the tall tiles the wide one.  (Small tiles of weight
+    classes into an odd multiple of 96 columns read none.)"""
     g = tile_geometry(dtype, ntaps=ntaps, n_out=n_out, cin=cin, cout=cout, q8=q8,
                       class_rows=class_rows, epi_mode=epi_mode)
     return geometry_section(g)
@@ -508,7 +509,8 @@ def set_tile_geometry(geometry: int) -> None:
     """spc_conv_set_tile_geometry: TILES_WIDE / TILES_SMALL / TILES_TALL /
     TILES_LONG force the conv kernel's tile geometry for every later conv of the
     process (where it applies); TILES_AUTO (the default) lets each conv pick
-    by shape.  Results are the same."""
+    by shape.  Results are the same (the norm epilogue's may differ by a
+    rounding: by shape, few rows run it as a row pass)."""
     _check("spc_conv_set_tile_geometry", lib().spc_conv_set_tile_geometry(int(geometry)))
 
 

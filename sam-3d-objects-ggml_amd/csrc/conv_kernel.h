@@ -407,7 +407,7 @@ struct TileLds {
     uint32_t* scratch;  // the geometry's SCRATCH words: dedupe bitmap + word ranks, or the hash
     uint16_t* sidx;     // (NTAPS + 1) x TM slot keys; row NTAPS = the zero slot
     uint32_t* tlw;      // kTapWords
-    int32_t* urow;      // UMAX source rows of the union slots
+    int32_t* urow;      // UCAP source rows of the union slots
     int32_t* srow;      // TM output rows of the tile rows
     int32_t* wsum;      // one per wave
     int32_t* misc;      // [0] tap mask [1] min source row [2] unused [3] U [4] fast
@@ -751,7 +751,7 @@ __global__ __launch_bounds__(512) void conv_plan_kernel(ConvArgs a, char* plan, 
 }
 
 // Workgroups per CU a geometry is built for: GeoWide and GeoQuad fill the
-// CU's LDS with one; GeoSmall's ~42 KB and GeoTall's ~53 KB admit three (register
+// CU's LDS with one; GeoSmall's ~46 KB and GeoTall's ~53 KB admit three (register
 // budget 168 per wave), two for 128-column tiles, whose 64 x 64 wave tiles
 // need ~226 registers.
 template <typename GEO, int TN>
@@ -2086,7 +2086,9 @@ hipError_t dispatch_tn(hipStream_t s, const ConvArgs& a) {
     // a ragged last round of 128-column tiles (e.g. 368 tiles on 256 compute
     // units: two rounds, the second 44% full) costs a whole round; 64-column
     // tiles (about 0.6 of the time each) pay off when they need fewer than
-    // 10/6 as many rounds (SubM 1024 -> 1024 over 11774 rows: 627 -> 591 us)
+    // 10/6 as many rounds (wide SubM tiles 1024 -> 1024 over 11774 rows: 627 ->
+    // 591 us).  By shape this meets the 1 x 1 x 1 conv, weight classes and
+    // unpacked weights: packed 27-tap convs with such a round take small tiles.
     if constexpr (!Q8) {
         if (tn == 128) {
             const int64_t r128 = ceil_div(tiles_m * (a.cout / 128), a.num_cu);
@@ -2099,7 +2101,10 @@ hipError_t dispatch_tn(hipStream_t s, const ConvArgs& a) {
     // one 192-column tile of 4 waves (2 x 2, 128x96 wave tiles, one per
     // SIMD) instead of three 64-column tiles of 64x32 wave tiles, which read
     // each A fragment for half the MFMA work and are LDS-bound.  Packed
-    // 16-bit weights, and only once the row tiles alone fill the device.
+    // 16-bit weights, and only once the row tiles alone fill the device.  By
+    // shape these are the 1 x 1 x 1 convs: with 27 taps and with weight classes
+    // the small and the class tiles take such sizes (their rules hold both
+    // sides' times), and the wide ones run where that geometry is forced.
     if constexpr (!Q8 && PACKED && sizeof(T) == 2) {
         if (a.cout % 192 == 0 && a.cout % 128 != 0 && a.epi_mode != SPC_EPI_NORM_MOD_SILU &&
             tiles_m * (a.cout / 192) >= a.num_cu)

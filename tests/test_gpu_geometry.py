@@ -1,8 +1,8 @@
-"""The conv kernel's three tile geometries (SPC_TILES_WIDE: 256-row tiles over
-a double-buffered 895-row stage; SPC_TILES_SMALL: 128-row tiles, 64 for 8
-taps, over a single 511-row stage, several workgroups per CU;
+"""The conv kernel's four tile geometries (SPC_TILES_WIDE: 256-row tiles over
+a double-buffered 895-row stage; SPC_TILES_SMALL: 128-row tiles over a single
+575-row stage, 64 over 511 for 8 taps, several workgroups per CU;
 SPC_TILES_TALL: 256-row tiles over a single 559-row stage, reading the wide
-plan) compute every output row with the same sequence of MFMA steps --
+plan; SPC_TILES_LONG: 320-row tiles over a 1119-row stage) compute every output row with the same sequence of MFMA steps --
 chunks outer, active taps ascending, absent taps adding exact zeros -- so
 their outputs are equal value for value, with and without a tile plan, for
 every dtype, epilogue and staging path.  The small and the tall tiles are
@@ -268,9 +268,9 @@ def test_q8_0_wide_equals_small(spc, orc, dev, geo):
 
 def test_wide_span_and_fallback_small(spc, orc, dev, geo):
     """Small tiles whose sources span beyond the bitmap window (the LDS hash
-    dedupe) and tiles in random row order (union beyond the 511-row stage:
+    dedupe) and tiles in random row order (union beyond the 575-row stage:
     the per-tap fallback) equal the wide tiles; so do the tall tiles (the
-    shuffled shell's 256-row unions exceed their 511-row stage too)."""
+    shuffled shell's 256-row unions exceed their 559-row stage too)."""
     import torch
 
     nat = geo
@@ -585,7 +585,8 @@ def test_small_96_192_tiles_equal_wide(spc, dev, geo, dt, cin, cout, n):
     """The small tiles of 96 and 192 columns (128 rows, weights two steps
     ahead) and, for the 8-tap weight classes, their in-kernel setup, against
     the wide ones value for value: row remainders, one chunk and several, a
-    tile past the 511-row stage (the per-tap fallback), plain and residual."""
+    first tile past the stage (575 rows; 511 for the classes: the per-tap
+    fallback) and others within it, plain and residual."""
     import torch
 
     nat = geo
@@ -612,8 +613,15 @@ def test_small_96_192_tiles_equal_wide(spc, dev, geo, dt, cin, cout, n):
     w8 = nat.pack_weights(r(24, cout, cin, std=0.1), layout=nat.W_TCK)
     idx8 = torch.randint(-20, 300, (768, 8), generator=g, device=dev, dtype=torch.int32)
     idx8[:128] = torch.randint(0, n_in, (128, 8), generator=g, device=dev, dtype=torch.int32)
-    perm = torch.randperm(768, generator=g, device=dev).to(torch.int32)
+    # rows permuted within their 128-row class tile: the scattered ones fill the first
+    perm = torch.cat([128 * k + torch.randperm(128, generator=g, device=dev)
+                      for k in range(6)]).to(torch.int32)
     perm[perm >= 700] = -1
+    unions = [int(torch.unique(t[t >= 0]).numel()) for t in
+              (idx8[p[p >= 0].long()] for p in perm.split(128))]
+    assert unions[0] > 511 and max(unions[1:]) <= 511
+    if n >= 128:
+        assert int(torch.unique(idx[:128][idx[:128] >= 0]).numel()) > 575
     ys = []
     for gm in (nat.TILES_WIDE, nat.TILES_SMALL):
         nat.set_tile_geometry(gm)
@@ -622,6 +630,44 @@ def test_small_96_192_tiles_equal_wide(spc, dev, geo, dt, cin, cout, n):
                                class_rows=256, n_classes=3)[:700] for p in (None, plan)]
     torch.cuda.synchronize()
     assert all(torch.equal(ys[0], y) for y in ys)
+
+
+@pytest.mark.parametrize("cin,cout", [(32, 64), (128, 128), (96, 96)])
+def test_small_stage_edges(spc, dev, geo, cin, cout):
+    """128-row tiles of exactly 511, 512, 575 and 576 source rows (the last past
+    the 27-tap stage, the second past the class tiles') against the wide ones."""
+    import torch
+
+    nat = geo
+    print(f"[case] small stage edges {cin}->{cout}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(cin)
+    r = lambda *s, std=1.0: (torch.randn(s, generator=g, device=dev) * std).bfloat16()  # noqa: E731
+    sizes = [511, 512, 575, 576]
+    n = 128 * len(sizes)
+
+    def table(ntaps):
+        rows = []
+        for k, u in enumerate(sizes):
+            t = torch.randint(0, u, (128, ntaps), generator=g, device=dev, dtype=torch.int32)
+            t.view(-1)[:u] = torch.arange(u, device=dev, dtype=torch.int32)
+            rows.append(t + 100 * k)
+        return torch.cat(rows).contiguous()
+
+    x, b = r(1000, cin), r(cout)
+    w, w8 = nat.pack_weights(r(cout, 27, cin, std=0.05)), nat.pack_weights(
+        r(16, cout, cin, std=0.1), layout=nat.W_TCK)
+    idx, idx8 = table(27), table(8)
+    assert [int(torch.unique(t).numel()) for t in idx8.split(128)] == sizes
+    ys, y8 = [], []
+    for gm in (nat.TILES_WIDE, nat.TILES_SMALL):
+        nat.set_tile_geometry(gm)
+        plan = nat.conv_plan(idx.view(-1), ntaps=27, n_out=n, n_in=1000)
+        ys += [nat.sparse_conv(x, w, b, idx.view(-1), ntaps=27, n_out=n, plan=p)
+               for p in (None, plan)]
+        y8.append(nat.sparse_conv(x, w8, b, idx8.view(-1), ntaps=8, n_out=n, class_rows=256,
+                                  n_classes=2))
+    torch.cuda.synchronize()
+    assert all(torch.equal(ys[0], y) for y in ys) and torch.equal(y8[0], y8[1])
 
 
 def test_small_tile_rules(spc, dev, geo):
