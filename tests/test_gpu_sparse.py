@@ -187,6 +187,38 @@ def test_stride2_module(spc, orc, dev):
         assert np.all(cb[sl] == i)
 
 
+def test_stride2_layout_follows_the_coordinates(spc, dev):
+    """The coarse batch slices kept with the map: a caller's list is its own,
+    and new coordinates (another tensor, or the same one rewritten) have new
+    slices."""
+    import torch
+
+    sp = _sp(spc)
+    sets = [torch.from_numpy(spc.workloads.random_voxels(k, 12, batches=3, seed=s)).to(dev)
+            for k, s in ((900, 1), (900, 2))]
+    n = min(c.shape[0] for c in sets)
+    a, b = (c[:n].contiguous() for c in sets)
+    conv = sp.SparseConv3d(32, 32, 2, stride=2).to(dev)
+    _case(f"stride-2 layout N={n}")
+
+    def check(y):
+        cb = y.coords[:, 0].cpu().numpy()
+        assert [sl.stop - sl.start for sl in y.layout] == [int((cb == i).sum()) for i in range(3)]
+        for i, sl in enumerate(y.layout):
+            assert np.all(cb[sl] == i)
+
+    with torch.no_grad():
+        x = sp.SparseTensor(torch.randn((n, 32), device=dev), a.clone(), torch.Size([3, 32]))
+        y = conv(x)
+        check(y)
+        y.layout.clear()
+        check(conv(x))
+        x.coords.copy_(b)
+        check(conv(x))
+        x.coords = a
+        check(conv(x))
+
+
 def test_inverse_conv_dense_brute_force(spc, dev):
     """SparseInverseConv3d after a stride-2 conv, against torch
     conv_transpose3d on the dense grid, sampled at the fine voxels."""
@@ -430,6 +462,62 @@ def test_slat_tables(spc, orc, dev):
     }
     for k, v in pairs.items():
         assert np.array_equal(getattr(t, k).cpu().numpy().reshape(v.shape), v), k
+
+
+def _check_slat_tables(spc, orc, dev, coords, res):
+    import torch
+
+    t = spc.tables.SlatTables.build(torch.from_numpy(coords).to(dev), res)
+    n = coords.shape[0]
+    tm, d = orc.conv_table_slat(coords), orc.downsample_map(coords)
+    tmc = orc.conv_table_slat(d["coarse_coords"])
+    om, mk, ar = orc.spconv_tables(tm, n)
+    omc, mkc, arc = orc.spconv_tables(tmc, d["nc"])
+    assert (t.nf, t.nc) == (n, d["nc"])
+    for k, v in {"conv_fine": tm, "conv_fine_spconv": om, "conv_fine_mask": mk,
+                 "conv_fine_argsort": ar, "conv_coarse": tmc, "conv_coarse_spconv": omc,
+                 "conv_coarse_mask": mkc, "conv_coarse_argsort": arc,
+                 "fine_to_coarse": d["fine_to_coarse"], "coarse_children": d["children"],
+                 "coarse_count": d["counts"], "coarse_coords": d["coarse_coords"]}.items():
+        assert np.array_equal(getattr(t, k).cpu().numpy().reshape(v.shape), v), k
+
+
+@pytest.mark.parametrize("res,objects,fine,coarse", [
+    (63, 4, True, True),       # dense, odd: the coarse grid is 32 wide
+    (1, 1, True, True),        # one voxel
+    (192, 1, False, True),     # hashed fine level, dense coarse one
+    (257, 3, False, False),    # hashed both, odd
+    (1024, 1, False, False), (2000, 2, False, False)])
+def test_slat_tables_lookups(spc, orc, dev, res, objects, fine, coarse):
+    """Every lookup the builder chooses between, per level, with several items
+    and odd resolutions, against the oracle."""
+    n = 1 if res == 1 else 3000
+    c = spc.workloads.random_voxels(n, min(res, 40), batches=objects, seed=res)
+    c[:, 1:] += res - min(res, 40)  # up to the last cell
+    _case(f"SlatTables.build res={res} objects={objects} N={c.shape[0]}")
+    dense = spc.tables._dense
+    assert (dense(objects, res, c.shape[0]) is not None) == fine
+    assert (dense(objects, (res + 1) // 2, c.shape[0]) is not None) == coarse
+    _check_slat_tables(spc, orc, dev, c, res)
+
+
+@pytest.mark.parametrize("res", [40, 300])  # dense, hashed
+@pytest.mark.parametrize("at,value", [((5, 1), "res"), ((0, 2), -1), ((7, 3), 1 << 20),
+                                      ((3, 0), -1)])
+def test_slat_tables_bad_coordinates(spc, orc, dev, res, at, value):
+    """A coordinate outside the resolution or a negative batch raises (the fine
+    build is queued before the check), and a good call after it is right."""
+    import torch
+
+    c = spc.workloads.random_voxels(500, 40, seed=2)
+    bad = c.copy()
+    bad[at] = res if value == "res" else value
+    _case(f"SlatTables.build bad coordinate {at} {value} res={res}")
+    with pytest.raises(spc._native.SparseConvError):
+        spc.tables.SlatTables.build(torch.from_numpy(bad).to(dev), res)
+    with pytest.raises(spc._native.SparseConvError):
+        spc.tables.SlatTables.build(torch.from_numpy(c - 41).to(dev), res)  # every batch negative
+    _check_slat_tables(spc, orc, dev, c, res)
 
 
 def test_slat_tables_resolution_forms(spc, dev):
