@@ -558,8 +558,9 @@ def _epilogue(x, n_out, cout, residual, norm_mod, residual_rows):
     if norm_mod is not None:
         scale, shift, coords, eps = norm_mod
         _need_gpu(scale, shift, coords)
-        scale = scale.to(torch.float32).contiguous()
-        shift = shift.to(torch.float32).contiguous()
+        if scale.dtype != torch.float32 or shift.dtype != torch.float32:
+            scale, shift = scale.to(torch.float32), shift.to(torch.float32)
+        scale, shift = scale.contiguous(), shift.contiguous()
         coords = coords.contiguous()
         if scale.shape != shift.shape or scale.dim() != 2 or scale.shape[1] != cout:
             raise ValueError("scale / shift must be [n_batch, cout]")
@@ -641,8 +642,9 @@ def sparse_conv(x: torch.Tensor, weight, bias: torch.Tensor | None,
 
 
 def products_workspace(n_in: int, cout: int, device) -> torch.Tensor:
-    """The products buffer of sparse_conv_products over n_in source rows."""
-    return _workspace(lib().spc_conv_products_workspace_bytes(n_in, cout), device)
+    """The products buffer of sparse_conv_products over n_in source rows
+    (spc_conv_products_workspace_bytes: 27 F32 products a row and column)."""
+    return _workspace(108 * n_in * cout, device)
 
 
 def sparse_conv_products(x: torch.Tensor, weight: PackedWeights, bias: torch.Tensor | None,

@@ -574,7 +574,9 @@ class _ConvCore:
         b = self.conv.bias
         if b is None:
             return None
-        b = b.detach().to(device=device, dtype=dtype)
+        b = b.detach()
+        if b.dtype != dtype or b.device != device:
+            b = b.to(device=device, dtype=dtype)
         cout_p = _pad32(self.conv.out_channels)
         if cout_p != b.shape[0]:
             b = torch.nn.functional.pad(b, (0, cout_p - b.shape[0]))
