@@ -1945,11 +1945,15 @@ hipError_t dispatch_small(hipStream_t s, const ConvArgs& a) {
 // For 16-bit weights the 128-, 192- and 96-column tiles choose by what the last
 // round of the CUs holds (t: tiles of 256 rows; us, wide / small):
 //   128  two small workgroups a CU run half rounds, so they gain while the last
-//        wide round is at most half full, and lose the wide tiles' overlapped
-//        staging where it is fuller: 1024 -> 1024 at t / CUs 1.06 501 / 449,
-//        1.47 577 / 530, 1.62 605 / 643, 1.91 640 / 676, 2.41 926 / 849,
-//        2.62 931 / 985, 3.41 1268 / 1190, 3.81 1291 / 1332; 256 -> 256 the
-//        same way; 128 -> 512 within 1 % above the half.
+//        wide round is at most half full, and over rows of more than four
+//        chunks lose the wide tiles' overlapped staging where it is fuller:
+//        1024 -> 1024 at t / CUs 1.06 501 / 449, 1.47 577 / 530, 1.62 605 / 655,
+//        1.81 630 / 672, 2.31 944 / 861, 2.62 946 / 1004, 3.62 1284 / 1335; 256 ->
+//        256 the same way (1.6 161 / 171, 2.6 252 / 263), 192 -> 128 1.6 125 / 131,
+//        2.6 193 / 200.  Up to four chunks the fuller half is a draw in row order
+//        (128 -> 128 1.6 87 / 90, 1.8 91 / 93, 2.8 139 / 140; 96 -> 128 1.8 72 / 72)
+//        and rows in random order, which take the per-tap fallback, prefer the
+//        small ones (128 -> 128 1.6 302 / 289; 128 -> 256 288 / 272).
 //   192  as soon as three 64-column wide tiles a row tile need a third round
 //        (t above 2/3 CUs): 192 -> 192 at 0.3 40 / 56, 0.6 77 / 88, 0.95 117 /
 //        97, 1.1 192 / 140, 1.7 197 / 182, 2.5 296 / 237, 6.2 719 / 597; 384 ->
@@ -1957,7 +1961,10 @@ hipError_t dispatch_small(hipStream_t s, const ConvArgs& a) {
 //   96   three a CU, above half a round: 96 -> 96 at 0.3 17 / 20, 0.6 31 / 27,
 //        0.95 46 / 31, 1.7 60 / 57, 2.5 92 / 72, 6.2 217 / 172; 32 -> 96 at 6.2
 //        96 / 70; 192 -> 96 at 0.3 28 / 35, 0.6 54 / 50, 1.7 107 / 106, 6.2 362 /
-//        322.
+//        322.  Not over more than four chunks in the fuller half of the second
+//        round, where wide tiles are full and three small rounds are not: 288 ->
+//        288 at 1.45 148 / 116, 1.54 145 / 153, 1.8 153 / 156, 2.2 219 / 182; 480 ->
+//        480 1.54 231 / 252, 1.95 255 / 273, 2.6 363 / 356; 192 -> 96 1.53 100 / 103.
 inline bool first_half_round(int64_t t, int64_t per_round) {
     const int64_t last = t % per_round;
     return last > 0 && 2 * last <= per_round;
@@ -1979,12 +1986,15 @@ bool use_small_tiles(const ConvArgs& a) {
         const int64_t tiles_m = ceil_div(a.n_out, GeoWide::TM);
         if constexpr (!Q8 && sizeof(T) == 2) {
             if (a.cout % 192 == 0 && a.cout % 128 != 0) return 3 * tiles_m * (a.cout / 192) > 2 * a.num_cu;
-            if (a.cout % 96 == 0 && a.cout % 64 != 0) return 2 * tiles_m * (a.cout / 96) > a.num_cu;
+            if (a.cout % 96 == 0 && a.cout % 64 != 0) {
+                const int64_t t = tiles_m * (a.cout / 96);
+                return 2 * t > a.num_cu && !(kch > 4 && 2 * t > 3 * a.num_cu && t <= 2 * a.num_cu);
+            }
         }
         if (kch <= 2) return a.cout <= 64;
         const int64_t t = tiles_m * (a.cout / 128);
         if (a.cout % 128 != 0 || t <= a.num_cu) return false;
-        return Q8 || sizeof(T) != 2 || first_half_round(t, a.num_cu);
+        return Q8 || sizeof(T) != 2 || kch <= 4 || first_half_round(t, a.num_cu);
     }
 }
 
@@ -2011,7 +2021,8 @@ bool use_tall_tiles(const ConvArgs& a) {
 // whose 256-row tiles need a second round of the CUs that the 320-row ones
 // do not -- otherwise a round for the last few tiles.  66,779 rows C 128, bf16:
 // 73.8 -> 57.4 us (small tiles before), with the norm epilogue 113 -> 71.5
-// (wide tiles in two rounds); 79,659 rows 71.3 -> 56.6; C_in 256, 131 -> 94.
+// (wide tiles in two rounds); 79,659 rows 71.3 -> 56.6; C_in 256, 131 -> 94; 64,
+// 48.8 -> 32.1; 32, 31.3 -> 21.6; 65,537 rows 51.3 / 51.5.
 // Forced (SPC_TILES_LONG), any packed 16-bit 27-tap conv whose C_out is a
 // multiple of 128, except Q8_0 and weight classes.
 template <typename T, bool Q8, bool PACKED, int NTAPS>
@@ -2102,9 +2113,9 @@ hipError_t dispatch_tn(hipStream_t s, const ConvArgs& a) {
     // SIMD) instead of three 64-column tiles of 64x32 wave tiles, which read
     // each A fragment for half the MFMA work and are LDS-bound.  Packed
     // 16-bit weights, and only once the row tiles alone fill the device.  By
-    // shape these are the 1 x 1 x 1 convs: with 27 taps and with weight classes
-    // the small and the class tiles take such sizes (their rules hold both
-    // sides' times), and the wide ones run where that geometry is forced.
+    // shape the 1 x 1 x 1 convs run these, with 27 taps the 96-column ones where
+    // use_small_tiles leaves them; other sizes take the small and the class tiles
+    // (their rules hold both sides' times) unless the wide geometry is forced.
     if constexpr (!Q8 && PACKED && sizeof(T) == 2) {
         if (a.cout % 192 == 0 && a.cout % 128 != 0 && a.epi_mode != SPC_EPI_NORM_MOD_SILU &&
             tiles_m * (a.cout / 192) >= a.num_cu)

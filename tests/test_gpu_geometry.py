@@ -686,3 +686,19 @@ def test_small_tile_rules(spc, dev, geo):
     assert [k(t, 192, 96, 8, 256 * t) for t in (128, 129)] == [W, S]
     assert [k(t, 768, 192, 8, 256 * t) for t in (170, 171)] == [W, S]
     assert k(300, 192, 192, dt=torch.float32) == W
+
+
+def test_small_tile_rules_by_chunks(spc, dev, geo):
+    """Rows of more than four 64-byte chunks leave the fuller half of a round of
+    128-column tiles, and of the second of 96-column ones, to the wide tiles."""
+    import torch
+
+    nat = geo
+    k = lambda t, cin, cout: nat.tile_geometry(  # noqa: E731
+        torch.bfloat16, ntaps=27, n_out=256 * t, cin=cin, cout=cout)
+    S, W = nat.TILES_SMALL, nat.TILES_WIDE
+    assert [k(t, 160, 256) for t in (128, 129, 192, 193, 256, 257)] == [W, S, S, W, W, S]
+    assert [k(t, 128, 256) for t in (128, 129, 192, 193, 256, 257)] == [W, S, S, S, S, S]
+    assert [k(t, 160, 96) for t in (128, 129, 384, 385, 512, 513, 700)] == [W, S, S, W, W, S, S]
+    assert [k(t, 128, 96) for t in (128, 129, 384, 385, 512, 513)] == [W, S, S, S, S, S]
+    assert [k(t, 288, 288) for t in (42, 43, 128, 129, 170, 171)] == [W, S, S, W, W, S]
