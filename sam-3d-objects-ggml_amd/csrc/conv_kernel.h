@@ -78,7 +78,7 @@ struct ConvArgs {
     int32_t tiles_n;
     int32_t col_major;        // full row tiles' tiles taken column tile by column tile
     int64_t total_tiles;
-    int64_t heavy_tiles;      // tiles of full row tiles (mapped XCD-major)
+    int64_t heavy_tiles;      // tiles mapped XCD-major: of the full row tiles, or all
     int64_t class_rows;       // > 0: rows [c * class_rows, (c + 1) * class_rows) use weight
     int32_t n_classes;        //   taps c * ntaps .. (packed weights of n_classes * ntaps taps)
     int64_t tiles_per_xcd;
@@ -838,11 +838,8 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
 
     // Tile mapping: the tiles of the full row tiles XCD-major (workgroup b
     // runs on XCD b % 8, each XCD gets a contiguous range of them), then the
-    // tiles of a partial last row tile, which run last: first in the places
-    // that the last XCDs' ranges leave over, so that as many tiles as CUs are
-    // one round (behind every XCD's range they were a second one on XCD 0:
-    // 81,500 rows C 128 in 320-row tiles 87 -> 57 us, 32,500 rows
-    // 512 -> 128 with the norm row pass 166 -> 111, 129,761 rows 256 -> 128 216 -> 176).
+    // tiles of a partial last row tile, which run last and cost little (where
+    // they would cost a round, launch_conv counts them to the ranges).
     // Within the range, row tile by row tile (the column tiles of a row
     // tile share its gathered rows in the XCD's L2), or, with weights larger
     // than half an L2 (col_major), column tile by column tile: the tiles an
@@ -854,14 +851,15 @@ __global__ __launch_bounds__(WM * WN * 64, (geo_blocks_per_cu<GEO, TN>())) void 
         const int64_t xcd = blockIdx.x & 7;
         const int64_t local = blockIdx.x >> 3;
         tile = xcd * a.tiles_per_xcd + local;
-        if (tile >= a.total_tiles) return;
+        if (tile >= a.heavy_tiles) return;
     } else {
-        tile = blockIdx.x;
+        tile = a.heavy_tiles + ((int64_t)blockIdx.x - hb);
+        if (tile >= a.total_tiles) return;
     }
     int64_t tm;
     int tn;
     if (tile < a.heavy_tiles && a.col_major) {
-        const int64_t mfull = a.heavy_tiles / a.tiles_n;  // full row tiles
+        const int64_t mfull = a.heavy_tiles / a.tiles_n;  // row tiles of the ranges
         tm = tile % mfull;
         tn = (int)(tile / mfull);
     } else {
@@ -1846,7 +1844,17 @@ hipError_t launch_conv(hipStream_t s, ConvArgs a) {
     a.tiles_per_xcd = ceil_div(a.heavy_tiles, 8);
     const int64_t wbytes = (int64_t)NTAPS * max(1, a.n_classes) * a.cin * a.cout * (Q8 ? 1 : (int)sizeof(T));
     a.col_major = a.tiles_n > 1 && wbytes > (2 << 20);
-    const int64_t grid = a.tiles_per_xcd * 8 > a.total_tiles ? a.tiles_per_xcd * 8 : a.total_tiles;
+    // The partial row tile's tiles run behind the XCDs' ranges, unless they would
+    // begin another round of the CUs there: then they take the places that the
+    // ranges leave over (us: 81,500 rows C 128 in 320-row tiles 87 -> 57; 32,500
+    // rows 512 -> 128 with the norm row pass 166 -> 111; 129,761 rows 256 -> 128
+    // 216 -> 176).
+    const int64_t light = a.total_tiles - a.heavy_tiles;
+    const int64_t round = (int64_t)max(1, a.num_cu / 8) * geo_blocks_per_cu<GEO, TN>();  // places on an XCD
+    if (light <= a.tiles_per_xcd * 8 - a.heavy_tiles &&
+        ceil_div(a.tiles_per_xcd + ceil_div(light, 8), round) > ceil_div(a.tiles_per_xcd, round))
+        a.heavy_tiles = a.total_tiles;
+    const int64_t grid = a.tiles_per_xcd * 8 + (a.total_tiles - a.heavy_tiles);
     if (grid == 0) return hipSuccess;
     if (a.epi_mode == SPC_EPI_NORM_MOD_SILU && !norm_epilogue_fits<GEO, TN>())
         return hipErrorInvalidValue;  // the tile cannot hold the epilogue's rows

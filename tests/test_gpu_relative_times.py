@@ -43,14 +43,20 @@ def test_partial_tile_takes_no_round_of_its_own(spc, dev, n, whole, cin, cout, n
     w = (torch.randn((cout, 27, cin), generator=g, device=dev) * (27 * cin) ** -0.5).bfloat16()
     b = torch.randn(cout, generator=g, device=dev).bfloat16()
     pw, mod, us = nat.pack_weights(w), torch.zeros((12, cout), device=dev), []
-    for rows in (n, whole):
+    for rows in (n, whole):  # (the mapping's outputs against another geometry's, too)
         coords = torch.from_numpy(np.ascontiguousarray(c[:rows])).to(dev)
         m = nat.map_build(coords, outputs="token")
         p = nat.conv_plan(m.token_major, ntaps=27, n_out=rows)
         x = torch.randn((rows, cin), generator=g, device=dev).bfloat16()
-        us.append(_us(lambda: nat.sparse_conv(
-            x, pw, b, m.token_major, ntaps=27, n_out=rows, plan=p,
-            norm_mod=(mod, mod, coords, 1e-6) if norm else None), 30))
+        run = lambda nm=None: nat.sparse_conv(x, pw, b, m.token_major, ntaps=27,  # noqa: E731
+                                              n_out=rows, plan=p, norm_mod=nm)
+        y = run()
+        nat.set_tile_geometry(nat.TILES_SMALL)
+        try:
+            assert torch.equal(y, run())
+        finally:
+            nat.set_tile_geometry(nat.TILES_AUTO)
+        us.append(_us(lambda: run((mod, mod, coords, 1e-6) if norm else None), 30))
     print(f"[time] {us[0]:.1f} / {us[1]:.1f} us", flush=True)
     assert us[0] <= 1.2 * us[1], us
 
